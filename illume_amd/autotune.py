@@ -7,9 +7,11 @@ triangles: exact distance ties go to the smaller instance and primitive). The tu
 measures time.
 
     bvh_layout       0: FP32 BVH2 nodes, 1: 8-bit BVH4 nodes (both are resident for every scene)
-    extend_mode      1: each wave traces one batch of 64 rays to completion
+    extend_mode      0: idle lanes refill after every traversal step; short queues are finished in
+                        one launch, four lanes per ray
+                     1: each wave traces one batch of 64 rays to completion
                      2: idle lanes refill from a wave-local queue at BLAS leaves
-                     3 (and 0, the default): idle lanes refill after every traversal step
+                     3: as 0, without the launch that finishes short queues
     refill_min       idle lanes that trigger a refill (modes 1 and 2)
     ext_fetch        rays an extend wave reserves from the queue at a time (work-queue granularity)
     leaf_wait_pct    per-step refill: lanes waiting at BLAS leaves (as a percentage of the other
@@ -39,7 +41,7 @@ DEFAULT_SPACE = (
     ("bvh_layout", (0, 1)),
     ("sample_group", (1, 4, 16, 64)),
     ("tile_rows", (1, 4, 8)),
-    (("extend_mode", "refill_min"), ((1, 0), (2, 16), (2, 32), (3, 8), (3, 16), (3, 32), (3, 48))),
+    (("extend_mode", "refill_min"), ((1, 0), (2, 16), (2, 32), (0, 8), (0, 16), (0, 32), (0, 48))),
     ("leaf_wait_pct", (40, 50, 60, 80, 100, 150)),
     ("shade_sort", (1, 2)),
     ("camera_packets", (1, 2)),

@@ -223,6 +223,55 @@ Layout2 make_layout2(const Tree& t) {
     return L;
 }
 
+LayoutF make_layout_f(const std::vector<BNode>& nodes, int root) {
+    LayoutF L;
+    L.root = root;
+    if (root < 0 || root == ILM_NO_CHILD) return L;
+    struct Kid { float4 a; float lz, hz; int code; double area; };
+    auto kid = [&nodes](int n, int k) {
+        const BNode& b = nodes[n];
+        Kid c;
+        if (k == 0) { c.a = b.a; c.lz = b.b.x; c.hz = b.b.y; c.code = b.d.x; }
+        else { c.a = make_float4(b.b.z, b.b.w, b.c.x, b.c.y); c.lz = b.c.z; c.hz = b.c.w; c.code = b.d.y; }
+        const double dx = (double)c.a.y - c.a.x, dy = (double)c.a.w - c.a.z, dz = (double)c.hz - c.lz;
+        c.area = dx < 0 || dy < 0 || dz < 0 ? 0.0 : dx * dy + dy * dz + dz * dx;
+        return c;
+    };
+    /* breadth first, so that a node's children lie near one another */
+    std::vector<std::pair<int, int>> todo = {{root, 1}};   /* BNode, level; FNode ids in this order */
+    for (size_t i = 0; i < todo.size(); i++) {
+        L.levels = std::max(L.levels, todo[i].second);
+        std::vector<Kid> ch = {kid(todo[i].first, 0), kid(todo[i].first, 1)};
+        while (ch.size() < 4) {
+            int best = -1;
+            for (size_t k = 0; k < ch.size(); k++)
+                if (ch[k].code >= 0 && ch[k].code != ILM_NO_CHILD && (best < 0 || ch[k].area > ch[best].area)) best = (int)k;
+            if (best < 0) break;
+            const int n = ch[best].code;
+            ch[best] = kid(n, 0);
+            ch.insert(ch.begin() + best + 1, kid(n, 1));
+        }
+        FNode f;
+        std::memset(&f, 0, sizeof(f));
+        for (int k = 0; k < 4; k++) {
+            int code = ILM_NO_CHILD;
+            if (k < (int)ch.size()) {
+                code = ch[k].code;
+                if (code >= 0 && code != ILM_NO_CHILD) {
+                    todo.push_back({code, todo[i].second + 1});
+                    code = (int)todo.size() - 1;
+                }
+                f.c[k].a = ch[k].a;
+                f.c[k].b = make_float4(ch[k].lz, ch[k].hz, 0.0f, 0.0f);
+            }
+            std::memcpy(&f.c[k].b.z, &code, 4);
+        }
+        L.nodes.push_back(f);
+    }
+    L.root = 0;
+    return L;
+}
+
 static inline float q_deq(float o, int q, float s) { return o + (float)q * s; }
 
 void qnode_child_box(const QNode& n, int k, float lo[3], float hi[3]) {

@@ -69,6 +69,16 @@ struct LayoutQ {
 };
 LayoutQ make_layout_q(const Tree& t);
 
+/* FP32 BVH4 (FNode) collapsed from a BNode tree: each node takes the two children of a BNode and
+ * opens the inner one of largest area until it holds four. levels: FNodes on the longest path
+ * from the root (0 when the root is a leaf or absent). */
+struct LayoutF {
+    std::vector<FNode> nodes;
+    int root = ILM_NO_CHILD;
+    int levels = 0;
+};
+LayoutF make_layout_f(const std::vector<BNode>& nodes, int root);
+
 /* Largest child-box quantum of the 8-bit layout the traversal accepts (2^24): with
  * |1/d| <= 1e30 the kernel's per-node products quantum * (1/d) stay finite. */
 #define ILM_QUANT_MAX_EXP 24

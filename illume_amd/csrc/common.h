@@ -44,6 +44,18 @@ struct __attribute__((aligned(16))) QNode {
 };
 static_assert(sizeof(QNode) == 64, "QNode is one 64-byte line");
 
+/* FP32 BVH4 node, 128 B, for the walk with four lanes per ray (quad.h): lane k reads child k's
+ * 32 bytes, so a quad reads one line. Collapsed from the BNode tree; same child encoding. */
+struct __attribute__((aligned(128))) FNode {
+    struct Child {
+        float4 a;           /* lo.x hi.x lo.y hi.y */
+        float4 b;           /* lo.z hi.z child code bits, 0 */
+    } c[4];                 /* unused slots: code ILM_NO_CHILD */
+};
+static_assert(sizeof(FNode) == 128, "FNode is one 128-byte line");
+/* stack entries per quad of that walk; scenes with a larger bound are not given to it */
+#define ILM_QUAD_STACK 64
+
 #define ILM_NO_CHILD ((int32_t)0x7fffffff)
 #define ILM_LEAF_MAX 16
 __host__ __device__ inline int32_t ilm_leaf_code(uint32_t first, uint32_t count) {
@@ -103,8 +115,12 @@ struct DInst {
     const float* uv;
     const int* idx;
     const float* pos;
+    /* the BLAS as FNodes (bytes 176..191) */
+    const FNode* fnodes;
+    int froot;
+    int fpad;
 };
-static_assert(sizeof(DInst) == 176, "DInst is 11 16-byte words");
+static_assert(sizeof(DInst) == 192, "DInst is 12 16-byte words");
 #define ILM_INST_FACE_NORMALS 1
 #define ILM_INST_TEXCOORDS 2
 
@@ -118,6 +134,8 @@ struct DMesh {
     const float* uv;        /* 2 per vertex, or null */
     const float4* svert;    /* 3 per original triangle: its vertex normals, or with face normals its
                                vertex positions (w = 0), so shading reads them in one request */
+    const FNode* fnodes;
+    int froot;
     int root;               /* root child code (FP32 layout) */
     int qroot;              /* root child code (quantised layout) */
     int face_normals;
@@ -147,7 +165,9 @@ struct DScene {
     float cam[12];          /* rows 0..2 of the camera matrix */
     float dof;
     float aperture;
-    int pad[2];
+    int ftlas_root;
+    int pad;
+    const FNode* ftlas;     /* the TLAS as FNodes */
 };
 
 /* One request inside a launch. */
@@ -212,6 +232,9 @@ struct DChunk {
     DWork work[ILM_MAX_WORK];
 };
 
+/* Largest grid (one wave per workgroup) of k_finish. */
+#define ILM_TAIL_WAVES 8192
+
 /* Per-chunk control block (device). Cleared by k_ctl_init, never by a memset. */
 struct DCtl {
     uint32_t count[ILM_MAX_DEPTH + 2];   /* live paths entering depth d */
@@ -219,6 +242,7 @@ struct DCtl {
     unsigned long long segments;
     uint32_t total;
     uint32_t pad;
+    uint32_t tail[ILM_TAIL_WAVES];       /* segments each wave of k_finish traced */
 };
 
 /* Path state, struct of arrays; two copies ping-pong across depths. */
@@ -257,6 +281,8 @@ struct KParams {
     int cam0;               /* the first depth forms camera rays in extend and shade (no raygen) */
     int packet0;            /* ... and its extend traces each wave's camera rays as one packet */
     int uni_scene;          /* every request of the chunk renders the same scene */
+    int tail_only;          /* the whole chunk fits quad_max: no per-depth launches */
+    int quad_max;           /* queues of at most this many rays go to the quad walk (0: none) */
 };
 
 /* Path id order of a slice: local index l <-> (sample k of the slice, pixel slot q). Samples

@@ -31,6 +31,7 @@ struct ilm_scene {
     int64_t mesh_tris = 0;
     int stack_bound_fp32 = 0;
     int stack_bound_q = 0;
+    int stack_bound_f = 0;      /* quad walk over FNodes */
     int quant_max_exp = -127;   /* largest child-box quantum exponent of the 8-bit trees */
 };
 
@@ -127,7 +128,7 @@ struct ilm_ctx {
     hipStream_t copy_stream = nullptr;
     ilm_opts opts;
     int n_cu = 0;
-    int ext_grid = 0, shade_grid = 0, gen_grid = 0;
+    int ext_grid = 0, shade_grid = 0, gen_grid = 0, fin_grid = 0;
     int ovf_grid = 0;               /* extend grid the spill area (ovf) is sized for, >= ext_grid */
     std::chrono::steady_clock::time_point t0;
 

@@ -202,7 +202,7 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
     /* ---- meshes: BVH, layouts, triangle slots ---- */
     std::vector<DMesh> dmeshes(d->num_meshes);
     std::vector<Box> mesh_bounds(d->num_meshes);
-    int blas_depth = 0, blas_qdepth = 0;
+    int blas_depth = 0, blas_qdepth = 0, blas_flevels = 0;
     BuildOpts bo;
     for (int i = 0; i < d->num_meshes; i++) {
         const ilm_mesh_desc& m = d->meshes[i];
@@ -246,6 +246,10 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
         BNode* bn; QNode* qn; float4* tp; int* ip; float* pp; float* np; float* up;
         HIPTRY(ctx, dupload(s.get(), &bn, bvh.nodes.data(), bvh.nodes.size()));
         HIPTRY(ctx, dupload(s.get(), &qn, bvh.qnodes.data(), bvh.qnodes.size()));
+        const LayoutF lf = make_layout_f(bvh.nodes, bvh.root);
+        FNode* fn;
+        HIPTRY(ctx, dupload(s.get(), &fn, lf.nodes.data(), lf.nodes.size()));
+        blas_flevels = std::max(blas_flevels, lf.levels);
         HIPTRY(ctx, dupload(s.get(), &tp, tris.data(), tris.size()));
         HIPTRY(ctx, dupload(s.get(), &ip, m.indices, 3 * (size_t)m.num_triangles));
         HIPTRY(ctx, dupload(s.get(), &pp, m.positions, 3 * (size_t)m.num_vertices));
@@ -266,6 +270,8 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
         HIPTRY(ctx, dupload(s.get(), &svp, sv.data(), sv.size()));
         dm.nodes = bn; dm.qnodes = qn; dm.tris = tp; dm.idx = ip; dm.pos = pp; dm.nrm = np; dm.uv = up;
         dm.svert = svp;
+        dm.fnodes = fn;
+        dm.froot = lf.root;
         dm.root = bvh.root;
         dm.qroot = bvh.qroot;
         dm.face_normals = m.face_normals != 0;
@@ -295,6 +301,8 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
         di.uv = dmeshes[di.mesh].uv;
         di.idx = dmeshes[di.mesh].idx;
         di.pos = dmeshes[di.mesh].pos;
+        di.fnodes = dmeshes[di.mesh].fnodes;
+        di.froot = dmeshes[di.mesh].froot;
         di.flags = (d->meshes[di.mesh].face_normals ? ILM_INST_FACE_NORMALS : 0) |
                    (d->meshes[di.mesh].has_texcoords ? ILM_INST_TEXCOORDS : 0);
         for (int k = 0; k < 16; k++) {
@@ -325,8 +333,9 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
             ib.hi[a] = round_up(hi[a] + pad);
         }
     }
-    int tlas_depth = 0, tlas_qdepth = 0;
+    int tlas_depth = 0, tlas_qdepth = 0, tlas_flevels = 0;
     hs.tlas_root = ILM_NO_CHILD;
+    hs.ftlas_root = ILM_NO_CHILD;
     hs.qtlas_root = ILM_NO_CHILD;
     if (d->num_instances > 0) {
         BuildOpts to;
@@ -354,12 +363,20 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
         HIPTRY(ctx, dupload(s.get(), &qn, TQ.nodes.data(), TQ.nodes.size()));
         hs.tlas = bn; hs.qtlas = qn;
         hs.tlas_root = direct(T2.root);
+        const LayoutF tf = make_layout_f(T2.nodes, hs.tlas_root);
+        FNode* fn;
+        HIPTRY(ctx, dupload(s.get(), &fn, tf.nodes.data(), tf.nodes.size()));
+        hs.ftlas = fn;
+        hs.ftlas_root = tf.root;
+        tlas_flevels = tf.levels;
         hs.qtlas_root = direct(TQ.root);
     }
     /* device stack bound: pushes never exceed the depth of the current node per level */
     const int cap = ilm_k_lds_stack() + ilm_k_ovf_stack();
     s->stack_bound_fp32 = tlas_depth + 1 + blas_depth;
     s->stack_bound_q = 3 * (tlas_qdepth + 1) + 1 + 3 * (blas_qdepth + 1);
+    /* quad walk: a node leaves at most three entries, an instance entry one */
+    s->stack_bound_f = 3 * tlas_flevels + 1 + 3 * blas_flevels;
     if (s->stack_bound_fp32 > cap || (ctx->opts.bvh_layout == ILM_BVH_QUANT8 && s->stack_bound_q > cap))
         return fail(ctx, ILM_E_UNSUPPORTED, "BVH too deep for the traversal stack");
     if (ctx->opts.bvh_layout == ILM_BVH_QUANT8 && s->quant_max_exp > ILM_QUANT_MAX_EXP)
@@ -570,6 +587,7 @@ int ilm_open(int device, const ilm_opts* opts, ilm_ctx** out) {
     int occ = ilm_k_extend_occupancy(ctx->opts.tri_test, ctx->opts.bvh_layout, ext_mode_of(ctx->opts));
     ctx->ext_grid = ctx->n_cu * std::max(1, occ);
     ctx->gen_grid = ctx->n_cu * 8;
+    ctx->fin_grid = std::min(ILM_TAIL_WAVES, ctx->n_cu * ilm_k_finish_occupancy());
     /* 512-thread blocks, block-stride loop: one resident wave of blocks, no stragglers */
     ctx->shade_grid = ctx->n_cu * ilm_k_shade_occupancy(ctx->opts.shade_sort != 2);
     int rc = ctx_alloc_paths(ctx, cap_of(ctx->opts));
@@ -729,6 +747,13 @@ static bool scene_needs_ovf(const ilm_ctx* ctx, const ilm_scene* s) {
     const int bound = ctx->opts.bvh_layout == ILM_BVH_QUANT8 ? s->stack_bound_q : s->stack_bound_fp32;
     return bound > ilm_k_lds_stack();
 }
+/* whether the scene's FNode trees fit the quad walk's stacks */
+static bool scene_fits_quad(const ilm_scene* s) { return s->stack_bound_f <= ILM_QUAD_STACK; }
+static bool jobs_fit_quad(const std::vector<Job*>& jobs) {
+    for (const Job* j : jobs)
+        if (!scene_fits_quad(j->scene)) return false;
+    return true;
+}
 static bool jobs_need_ovf(const ilm_ctx* ctx, const std::vector<Job*>& jobs) {
     for (const Job* j : jobs)
         if (scene_needs_ovf(ctx, j->scene)) return true;
@@ -775,6 +800,25 @@ static KParams base_params(ilm_ctx* ctx, const Pipe& q) {
 }
 static KParams base_params(ilm_ctx* ctx) { return base_params(ctx, ctx_pipe(ctx)); }
 
+/* Queues of at most this many paths are finished by k_finish in one launch instead of two launches
+ * per remaining depth. A depth of a short queue costs the per-depth kernels some 110 us however
+ * few its paths are: the slowest of its walks, of one lane, and the launches (a 100k-triangle
+ * mesh, 1920x1080, 1 spp: 90 us per depth past the fifth). k_finish keeps 5120 waves of 64
+ * paths resident; past that a wave runs share after share, and its quads trace a long queue at
+ * 0.4 of the per-lane kernel's rate. Measured over limits of 50k to 1.4M: 320x240, 8 spp, depth 45
+ * in a medium 5.75 ms without, 3.49 at 50k, 2.82 at 200k, 2.76 at 330k, 3.06 at 700k; 960x720,
+ * 32 spp 27.9, 27.8, 27.0, 27.4, 30.6; 640x480, 32 spp, depth 16 5.63, 5.55, 5.03, 4.93, 5.13. */
+#define ILM_TAIL_PATHS (1 << 18)
+
+/* How this chunk's launches trace it: short queues go to k_finish when every scene's FNode trees
+ * fit its stacks (not while every depth's extend launch is timed or its tests counted, nor when
+ * the caller asked for an extend kernel by name). */
+static void chunk_choices(const ilm_ctx* ctx, uint32_t total_paths, bool quad_fits, KParams& P) {
+    const bool quad = quad_fits && ctx->opts.extend_mode == ILM_EXTEND_DEFAULT && !ctx->opts.profile && !ctx->opts.count_tests;
+    P.quad_max = quad ? ILM_TAIL_PATHS : 0;
+    P.tail_only = (int64_t)total_paths <= (int64_t)P.quad_max ? 1 : 0;
+}
+
 /* Stage a chunk descriptor: pinned ring slot -> the device DChunk dst (ordered on stream s). */
 static int stage_chunk(ilm_ctx* ctx, const DChunk& hc, DChunk* dst, hipStream_t s) {
     int slot = ctx->ring_pos++ % ILM_RING;
@@ -792,7 +836,7 @@ static int stage_chunk(ilm_ctx* ctx, const DChunk& hc, DChunk* dst, hipStream_t 
 static hipError_t start_paths(ilm_ctx* ctx, const Pipe& q, KParams& P, hipStream_t s) {
     P.in = q.A;
     P.cam0 = P.extend_mode == ILM_EXTEND_STEP_REFILL ? 1 : 0;
-    if (P.cam0 && P.packet0) return hipSuccess;
+    if (P.cam0 && (P.packet0 || P.tail_only)) return hipSuccess;
     return P.cam0 ? ilm_k_path_clear(P, ctx->gen_grid, s) : ilm_k_raygen(P, ctx->gen_grid, s);
 }
 
@@ -804,7 +848,7 @@ static int enqueue_depths(ilm_ctx* ctx, const Pipe& q, const KParams& base, int 
     KParams P = base;
     HIPTRY(ctx, ilm_k_ctl_init(P, s));
     HIPTRY(ctx, start_paths(ctx, q, P, s));
-    for (int d = 0; d < depth_steps; d++) {
+    for (int d = 0; d < (base.tail_only ? 0 : depth_steps); d++) {
         P.in = (d & 1) ? q.B : q.A;
         P.out = (d & 1) ? q.A : q.B;
         if (prof) {
@@ -820,11 +864,16 @@ static int enqueue_depths(ilm_ctx* ctx, const Pipe& q, const KParams& base, int 
         }
         HIPTRY(ctx, ilm_k_shade(P, d, ctx->shade_grid, s));
     }
+    if (base.quad_max > 0) {
+        P.in = q.A;
+        P.out = q.B;
+        HIPTRY(ctx, ilm_k_finish(P, ctx->fin_grid, s));
+    }
     return ILM_OK;
 }
 static int enqueue_finish(ilm_ctx* ctx, const Pipe& q, const KParams& base) {
     HIPTRY(ctx, ilm_k_accumulate(base, ctx->gen_grid, q.stream));
-    HIPTRY(ctx, ilm_k_chunk_end(base, q.seg_total, q.stream));
+    HIPTRY(ctx, ilm_k_chunk_end(base, q.seg_total, base.quad_max > 0 ? ctx->fin_grid : 0, q.stream));
     return ILM_OK;
 }
 /* both parts, on one stream (debug paths and the allocation-free render) */
@@ -867,7 +916,7 @@ static int run_graph(ilm_ctx* ctx, int key, const Pipe& q, const KParams& P, int
  * pipeline still runs; its accumulation waits for the previous chunk's (acc_ev of the other
  * pipeline) and for the latest clear of request buffers (fill_ev), so every pixel's sums grow
  * in pass order. Profiling and test counting keep one pipeline. Sets *pipe_used. */
-static int launch_chunk(ilm_ctx* ctx, const DChunk& hc, bool ovf, ProfileSink* prof, int* pipe_used = nullptr) {
+static int launch_chunk(ilm_ctx* ctx, const DChunk& hc, const std::vector<Job*>& jobs, ProfileSink* prof, int* pipe_used = nullptr) {
     const bool two = ctx->npipes == 2 && !prof && !ctx->opts.count_tests;
     const int k = two ? ctx->next_pipe : 0;
     if (two) ctx->next_pipe ^= 1;
@@ -875,19 +924,21 @@ static int launch_chunk(ilm_ctx* ctx, const DChunk& hc, bool ovf, ProfileSink* p
     int rc = stage_chunk(ctx, hc, q.chunk, q.stream);
     if (rc) return rc;
     KParams P = base_params(ctx, q);
+    const bool ovf = jobs_need_ovf(ctx, jobs);
     P.use_ovf = ovf ? 1 : 0;
     const bool uni = chunk_uni_scene(hc);
     P.uni_scene = uni ? 1 : 0;
+    chunk_choices(ctx, hc.total_paths, jobs_fit_quad(jobs), P);
     const int D = hc.depth_steps;
     const bool graphs = ctx->opts.use_graphs && !prof && !ctx->opts.count_tests;
-    if (graphs) rc = run_graph(ctx, 2 * (8 * D + 4 * k + (uni ? 2 : 0) + (ovf ? 1 : 0)), q, P, D, false);
+    if (graphs) rc = run_graph(ctx, 2 * (32 * D + 16 * (P.quad_max > 0) + 8 * P.tail_only + 4 * k + (uni ? 2 : 0) + (ovf ? 1 : 0)), q, P, D, false);
     else rc = enqueue_depths(ctx, q, P, D, prof);
     if (rc) return rc;
     if (ctx->npipes == 2) {
         HIPTRY(ctx, hipStreamWaitEvent(q.stream, ctx->acc_ev[k ^ 1], 0));
         if (k == 1) HIPTRY(ctx, hipStreamWaitEvent(q.stream, ctx->fill_ev, 0));
     }
-    if (graphs) rc = run_graph(ctx, 2 * k + 1, q, P, D, true);
+    if (graphs) rc = run_graph(ctx, 2 * (2 * (P.quad_max > 0) + k) + 1, q, P, D, true);
     else rc = enqueue_finish(ctx, q, P);
     if (rc) return rc;
     HIPTRY(ctx, hipEventRecord(ctx->acc_ev[k], q.stream));
@@ -1152,7 +1203,7 @@ static int run_jobs_sync(ilm_ctx* ctx, std::vector<Job*>& jobs, ilm_render_info*
         if (in_chunk.empty()) break;
         /* pass offsets: first_sample shifts every pass of the request */
         for (int w = 0; w < hc->n_work; w++) hc->work[w].pass0 += in_chunk[hc->work[w].req]->p.first_sample;
-        int rc = launch_chunk(ctx, *hc, jobs_need_ovf(ctx, in_chunk), ctx->opts.profile ? &prof : nullptr);
+        int rc = launch_chunk(ctx, *hc, in_chunk, ctx->opts.profile ? &prof : nullptr);
         if (rc) return rc;
         chunks++;
         max_paths = std::max<int64_t>(max_paths, hc->total_paths);
@@ -1379,6 +1430,7 @@ int ilm_render_noalloc(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* 
         P.trav_stats = nullptr;
         P.use_ovf = spill ? 1 : 0;
         P.uni_scene = 1;
+        chunk_choices(ctx, hc.total_paths, scene_fits_quad(scene), P);
         rc = enqueue_pipeline(ctx, q, P, hc.depth_steps, nullptr);
         if (rc) return rc;
         chunks++;
@@ -1443,7 +1495,10 @@ int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int
         P.trav_stats = nullptr;
         P.use_ovf = scene_needs_ovf(ctx, scene) ? 1 : 0;
         HIPTRY(ctx, ilm_k_ctl_init(P, ctx->stream));
-        HIPTRY(ctx, ilm_k_extend(P, 0, ctx->ovf, ctx->ext_grid, ctx->stream));
+        KParams F = P;
+        chunk_choices(ctx, (uint32_t)m, scene_fits_quad(scene), F);
+        if (F.tail_only) HIPTRY(ctx, ilm_k_extend_quad(P, 0, ctx->fin_grid, ctx->stream));
+        else HIPTRY(ctx, ilm_k_extend(P, 0, ctx->ovf, ctx->ext_grid, ctx->stream));
         h4.resize(m);
         hi.resize(m);
         HIPTRY(ctx, hipMemcpyAsync(h4.data(), ctx->hits.h, m * sizeof(float4), hipMemcpyDeviceToHost, ctx->stream));
@@ -1500,20 +1555,8 @@ int ilm_debug_path_radiance(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_par
         P.use_ovf = scene_needs_ovf(ctx, scene) ? 1 : 0;
         P.list = d_list;
         P.seg_count = ctx->seg_count;
-        if (ilm_k_ctl_init(P, ctx->stream) != hipSuccess || start_paths(ctx, ctx_pipe(ctx), P, ctx->stream) != hipSuccess) {
-            rc = fail(ctx, ILM_E_DEVICE, "raygen launch");
-            break;
-        }
-        for (int d = 0; d < params->max_depth; d++) {
-            P.in = (d & 1) ? ctx->B : ctx->A;
-            P.out = (d & 1) ? ctx->A : ctx->B;
-            if (ilm_k_extend(P, d, ctx->ovf, ctx->ext_grid, ctx->stream) != hipSuccess ||
-                ilm_k_shade(P, d, ctx->shade_grid, ctx->stream) != hipSuccess) {
-                rc = fail(ctx, ILM_E_DEVICE, "depth launch");
-                break;
-            }
-        }
-        if (rc) break;
+        chunk_choices(ctx, (uint32_t)m, scene_fits_quad(scene), P);
+        if ((rc = enqueue_depths(ctx, ctx_pipe(ctx), P, params->max_depth, nullptr))) break;
         c4.resize(m);
         sc.resize(m);
         if (hipMemcpyAsync(c4.data(), ctx->contrib, m * sizeof(float4), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
@@ -1604,7 +1647,7 @@ static void server_loop(ilm_ctx* ctx) {
                 build_chunk(ctx, issuable, *hc, in_chunk);
                 for (int w = 0; w < hc->n_work; w++) hc->work[w].pass0 += in_chunk[hc->work[w].req]->p.first_sample;
                 int pk = 0;
-                int rc = launch_chunk(ctx, *hc, jobs_need_ovf(ctx, in_chunk), nullptr, &pk);
+                int rc = launch_chunk(ctx, *hc, in_chunk, nullptr, &pk);
                 const Pipe q = ctx_pipe(ctx, pk);
                 Inflight f;
                 f.seg_slot = ctx->seg_ring_pos++ % ILM_RING;   /* at most two chunks in flight */

@@ -18,7 +18,7 @@
  * Every kernel reads its work count from device memory, so a whole chunk is a fixed launch
  * sequence (capturable as a hipGraph) with no host synchronisation between depths.
  */
-#include "traverse.h"
+#include "quad.h"
 
 #ifndef SHADE_BLOCK
 #define SHADE_BLOCK 512                       /* 8 waves share one compaction atomic */
@@ -34,6 +34,9 @@
 #define SHADE_BOUNDS __launch_bounds__(SHADE_BLOCK)
 #endif
 #define SHADE_WAVES (SHADE_BLOCK / 64)
+/* Waves per SIMD of k_finish (96 registers, no spills): the walk and the shading each need about
+ * 75. 4 and 6 waves measured within 1 % of 5 on queues that fit, 6 slower on the smallest. */
+#define FIN_WPE 5
 
 __global__ void k_ctl_init(DCtl* ctl_, const DChunk* chunk) {
     GLOBAL DCtl* ctl = gpw(ctl_);
@@ -428,6 +431,7 @@ __global__ SHADE_BOUNDS void k_shade(KParams P, int depth) {
     __shared__ uint32_t s_wk[OCT ? SHADE_WAVES * SHADE_KEYS : 1];
     GLOBAL DCtl* ctl = gpw(P.ctl);
     const uint32_t count = ctl->count[depth];
+    if (count <= (uint32_t)P.quad_max) return;   /* left to k_finish (every thread of the grid leaves) */
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
     const GLOBAL DReq* reqs = gp(P.chunk)->reqs;
@@ -550,6 +554,103 @@ __global__ SHADE_BOUNDS void k_shade(KParams P, int depth) {
     }
 }
 
+/* The rest of a chunk once a depth's queue is short (count <= P.quad_max; from there on the
+ * per-depth kernels leave the queue alone): every wave takes its share of the paths and carries
+ * them to their ends, segment after segment. Lane i owns path i of the wave's share: it stages
+ * its ray, the wave walks the live rays with four lanes each (quad_walk), and lane i shades its
+ * hit. A depth then costs a wave its own longest walk, not the whole queue's, and no launch. */
+template <int TRI, int UNI>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FIN_WPE, 8))) void k_finish(KParams P) {
+    __shared__ QuadLds lds;
+    LDSAS QuadLds* L = (LDSAS QuadLds*)&lds;
+    GLOBAL DCtl* ctl = gpw(P.ctl);
+    const int lane = threadIdx.x;
+    /* the first depth whose queue was left; its paths are in the buffers of that depth's parity */
+    const int D = uni_i(gp(P.chunk)->depth_steps);
+    int d0 = D;
+    uint32_t count = 0;
+    for (int b = 0; b < D; b += 64) {
+        const uint32_t c = b + lane < D ? ctl->count[b + lane] : 0xffffffffu;
+        const unsigned long long m = __ballot(c <= (uint32_t)P.quad_max);
+        if (m) {
+            const int k = (int)__builtin_ctzll(m);
+            d0 = b + k;
+            count = (uint32_t)__builtin_amdgcn_readlane((int)c, k);
+            break;
+        }
+    }
+    const bool swap = d0 & 1;
+    const GLOBAL float4* ino = gp(swap ? P.out.o : P.in.o);
+    const GLOBAL float4* ind = gp(swap ? P.out.d : P.in.d);
+    const GLOBAL float4* inc4 = gp(swap ? P.out.c : P.in.c);
+    const GLOBAL uint2* inr = gp(swap ? P.out.rng : P.in.rng);
+    const GLOBAL DReq* reqs = gp(P.chunk)->reqs;
+    const GLOBAL DScene* Su = UNI ? uni_p(gp(reqs[0].scene)) : nullptr;
+    uint32_t per = (count + gridDim.x - 1u) / gridDim.x;
+    per = per < 4u ? 4u : per > 64u ? 64u : per;
+    uint32_t segs = 0;
+    for (uint32_t base = blockIdx.x * per; base < count; base += gridDim.x * per) {
+        const uint32_t n0 = count - base < per ? count - base : per;
+        const uint32_t i = base + (uint32_t)lane;
+        bool live = (uint32_t)lane < n0;
+        V3 ro = mk3(0, 0, 0), rd = ro, color = mk3(1.0f, 1.0f, 1.0f);
+        uint64_t rs = 0;
+        uint32_t pixel = 0, pid = i;
+        int req = 0, medium = -1;
+        if (live) {
+            float4 o4, d4;
+            uint2 rg;
+            if (P.cam0 && d0 == 0) {
+                camera_ray(P, i, o4, d4, rg);
+                gpw(P.contrib)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (P.seg_count) gpw(P.seg_count)[i] = 0;
+            } else {
+                o4 = ino[i];
+                d4 = ind[i];
+                rg = inr[i];
+                const float4 c4 = inc4[i];
+                color = mk3(c4.x, c4.y, c4.z);
+                pid = f2u(c4.w);
+            }
+            ro = mk3(o4.x, o4.y, o4.z);
+            rd = mk3(d4.x, d4.y, d4.z);
+            req = (int)(f2u(o4.w) >> 16);
+            medium = (int)(f2u(o4.w) & 0xffffu) - 1;
+            pixel = f2u(d4.w);
+            rs = ((uint64_t)rg.y << 32) | (uint64_t)rg.x;
+        }
+        for (int depth = d0;; depth++) {
+            const unsigned long long lm = __ballot(live);
+            if (!lm) break;
+            const int n = __builtin_popcountll(lm);
+            segs += (uint32_t)n;
+            const int j = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(lm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)lm, 0u));
+            const GLOBAL DScene* S = UNI ? Su : gp(reqs[req].scene);
+            if (live)
+                quad_stage(L, j, S, ro, rd,
+                           medium_tmax(S, (uint32_t)(medium + 1), make_uint2((uint32_t)rs, (uint32_t)(rs >> 32)), pixel), req);
+            __syncthreads();
+            quad_walk<TRI, UNI>(L, n, reqs, Su);
+            __syncthreads();
+            if (live) {
+                const float4 h4 = make_float4(L->t[j], L->ray[0][j], L->ray[1][j], L->ray[2][j]);
+                const int hinst = L->inst[j];
+                const GLOBAL DReq* R = reqs + req;
+                ShadeRefs SR;
+                SR.inst = gp(S->inst);
+                SR.mats = gp(S->mats);
+                SR.mediums = gp(S->mediums);
+                if (P.seg_count) gpw(P.seg_count)[pid] += 1;
+                const int status = shade_path(S, SR, R->ray_bias, h4, hinst, ro, rd, color, medium, rs, ilm_pcg32_inc(pixel));
+                if (status == ST_EMIT) gpw(P.contrib)[pid] = make_float4(color.x, color.y, color.z, 0.0f);
+                live = status == ST_ALIVE && depth + 1 < R->max_depth;   /* src/renderer.cu:549 */
+            }
+            __syncthreads();
+        }
+    }
+    if (lane == 0) ctl->tail[blockIdx.x] = segs;
+}
+
 /* Kahan-compensated sum of the chunk's path radiances, pass order per pixel. One wave per
  * block takes 64 consecutive accumulate indices (pixels) at a time. Path ids come in runs of
  * `sgroup` passes per pixel, so when a wave's 64 pixels lie in one work item and the runs are at
@@ -637,12 +738,27 @@ __global__ __launch_bounds__(64) void k_accumulate(KParams P) {
     }
 }
 
-__global__ void k_chunk_end(DCtl* ctl, const DChunk* chunk, unsigned long long* seg_total) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        unsigned long long s = 0;
-        const int D = gp(chunk)->depth_steps;
-        for (int d = 0; d < D; d++) s += gp(ctl)->count[d];
-        gpw(ctl)->segments = s;
+/* Segments of the chunk: the queues the per-depth kernels traced (all of them, or with k_finish
+ * (tail_waves > 0) those longer than quad_max), and what k_finish's waves traced. */
+#define END_BLOCK 512
+__global__ __launch_bounds__(END_BLOCK) void k_chunk_end(DCtl* ctl_, const DChunk* chunk, unsigned long long* seg_total,
+                                                         int quad_max, int tail_waves) {
+    __shared__ unsigned long long part[END_BLOCK / 64];
+    GLOBAL DCtl* ctl = gpw(ctl_);
+    const int t = threadIdx.x;
+    const int D = gp(chunk)->depth_steps;
+    unsigned long long s = 0;
+    for (int d = t; d < D; d += END_BLOCK) {
+        const uint32_t c = ctl->count[d];
+        if (tail_waves == 0 || c > (uint32_t)quad_max) s += c;
+    }
+    for (int w = t; w < tail_waves; w += END_BLOCK) s += ctl->tail[w];
+    for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d);
+    if ((t & 63) == 0) part[t >> 6] = s;
+    __syncthreads();
+    if (t == 0) {
+        for (int w = 1; w < END_BLOCK / 64; w++) s += part[w];
+        ctl->segments = s;
         atomicAdd(gpw(seg_total), s);   /* chunks of the two pipelines may end together */
     }
 }
@@ -759,8 +875,23 @@ hipError_t ilm_k_accumulate(const KParams& P, int grid, hipStream_t s) {
     ILM_LAUNCH(k_accumulate, dim3(grid * 4), dim3(64), 0, s, P);
     return hipGetLastError();
 }
-hipError_t ilm_k_chunk_end(const KParams& P, unsigned long long* seg_total, hipStream_t s) {
-    ILM_LAUNCH(k_chunk_end, dim3(1), dim3(64), 0, s, P.ctl, P.chunk, seg_total);
+hipError_t ilm_k_extend_quad(const KParams& P, int depth, int grid, hipStream_t s) {
+    if (P.tri_test == ILM_TRI_WATERTIGHT) ILM_LAUNCH((k_extend_quad<1>), dim3(grid), dim3(64), 0, s, P, depth);
+    else ILM_LAUNCH((k_extend_quad<0>), dim3(grid), dim3(64), 0, s, P, depth);
+    return hipGetLastError();
+}
+hipError_t ilm_k_finish(const KParams& P, int grid, hipStream_t s) {
+    if (P.tri_test == ILM_TRI_WATERTIGHT) {
+        if (P.uni_scene) ILM_LAUNCH((k_finish<1, 1>), dim3(grid), dim3(64), 0, s, P);
+        else ILM_LAUNCH((k_finish<1, 0>), dim3(grid), dim3(64), 0, s, P);
+    } else {
+        if (P.uni_scene) ILM_LAUNCH((k_finish<0, 1>), dim3(grid), dim3(64), 0, s, P);
+        else ILM_LAUNCH((k_finish<0, 0>), dim3(grid), dim3(64), 0, s, P);
+    }
+    return hipGetLastError();
+}
+hipError_t ilm_k_chunk_end(const KParams& P, unsigned long long* seg_total, int tail_waves, hipStream_t s) {
+    ILM_LAUNCH(k_chunk_end, dim3(1), dim3(END_BLOCK), 0, s, P.ctl, P.chunk, seg_total, P.quad_max, tail_waves);
     return hipGetLastError();
 }
 hipError_t ilm_k_tonemap(const float4* accum, ilm_pixel* out, int n, int spp, int op, hipStream_t s) {
@@ -814,6 +945,7 @@ int ilm_k_shade_occupancy(int sort) {
                         : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_shade<0, 0>, SHADE_BLOCK, 0);
     return (e != hipSuccess || nb <= 0) ? 2 : nb;
 }
+int ilm_k_finish_occupancy() { return 4 * FIN_WPE; }
 int ilm_k_ovf_stack() { return OVF_STACK; }
 int ilm_k_lds_stack() { return LDS_STACK; }
 int ilm_k_ext_block() { return EXT_BLOCK; }

@@ -753,6 +753,16 @@ __device__ inline void packet_trace(const GLOBAL DScene* S, V3 O, V3 D, Best& B,
     }
 }
 
+/* Rays per reservation: `fetch`, or for a queue shorter than the grid's first reservations,
+ * about an even share of it in whole batches of 64, so that the rays spread over the waves
+ * instead of queueing behind one another in a few. */
+__device__ inline uint32_t pool_fetch(uint32_t count, uint32_t fetch) {
+    const uint32_t per = (count + gridDim.x - 1u) / gridDim.x;
+    const uint32_t share = per <= (uint32_t)EXT_BLOCK ? (uint32_t)EXT_BLOCK
+                                                      : (per + (uint32_t)(EXT_BLOCK - 1)) & ~(uint32_t)(EXT_BLOCK - 1);
+    return share < fetch ? share : fetch;
+}
+
 /* First depth with per-step refill: each wave reserves consecutive path ids (P.ext_fetch per
  * queue atomic, shrinking to 64 as the queue drains, as in k_extend), and traces them 64 at a
  * time: forms their camera rays (camera_ray) and walks one packet per distinct scene among them.
@@ -764,7 +774,8 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8)
     const int lane = threadIdx.x;
     GLOBAL DCtl* ctl = gpw(P.ctl);
     const uint32_t count = ctl->count[depth];
-    const uint32_t fetch = (uint32_t)P.ext_fetch;
+    if (count <= (uint32_t)P.quad_max) return;   /* left to k_finish */
+    const uint32_t fetch = pool_fetch(count, (uint32_t)P.ext_fetch);
     const GLOBAL DReq* reqs = gp(P.chunk)->reqs;
     TravCount tc = {0u, 0u};
     const uint32_t guide = gridDim.x * 2u;
@@ -987,15 +998,6 @@ __device__ inline bool seg_run(TState& T, Best& B, Stack<OVF>& st, const GLOBAL 
     }
 }
 
-/* Rays per reservation: `fetch`, or for a queue shorter than the grid's first reservations,
- * about an even share of it in whole batches of 64, so that the rays spread over the waves
- * instead of queueing behind one another in a few. */
-__device__ inline uint32_t pool_fetch(uint32_t count, uint32_t fetch) {
-    const uint32_t per = (count + gridDim.x - 1u) / gridDim.x;
-    const uint32_t share = per <= (uint32_t)EXT_BLOCK ? (uint32_t)EXT_BLOCK
-                                                      : (per + (uint32_t)(EXT_BLOCK - 1)) & ~(uint32_t)(EXT_BLOCK - 1);
-    return share < fetch ? share : fetch;
-}
 /* Work queue of the per-lane extend kernels: wave w first takes rays [w*fetch, (w+1)*fetch)
  * without an atomic, and the shared cursor then hands out what lies past the grid's first
  * reservations, `fetch` rays per atomic. A wave with no rays leaves without touching the cursor:
@@ -1296,6 +1298,7 @@ __global__ EXT_BOUNDS void k_extend_pers(KParams P, int depth, int* ovf_base) {
     st.sp = 0;
     GLOBAL DCtl* ctl = gpw(P.ctl);
     const uint32_t count = ctl->count[depth];
+    if (count <= (uint32_t)P.quad_max) return;   /* left to k_finish */
     const uint32_t fetch = pool_fetch(count, (uint32_t)P.ext_fetch);
     const GLOBAL float4* ino = gp(P.in.o);
     const GLOBAL float4* ind = gp(P.in.d);

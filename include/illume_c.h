@@ -179,7 +179,9 @@ typedef struct ilm_pixel {
 
 /* Extend-kernel scheduling (results are identical for every mode). BATCH: each wave traces 64
  * rays to completion; LEAF_REFILL: idle lanes take new rays when the wave reaches BLAS leaves;
- * STEP_REFILL: idle lanes take new rays after every traversal step (the default). */
+ * STEP_REFILL: idle lanes take new rays after every traversal step. DEFAULT: step refill for
+ * long queues; a queue of at most 2^18 paths is carried to its end in one launch, four lanes per
+ * ray. */
 enum { ILM_EXTEND_DEFAULT = 0, ILM_EXTEND_BATCH = 1, ILM_EXTEND_LEAF_REFILL = 2, ILM_EXTEND_STEP_REFILL = 3 };
 
 typedef struct ilm_opts {

@@ -1,0 +1,87 @@
+"""Queues of at most 2^18 paths are finished in one launch with four lanes per ray (the default
+extend mode): bit-identical to the per-depth kernels (extend_mode 3) whatever the path count."""
+import numpy as np
+import pytest
+
+import illume_amd
+import illume_amd.scenes as S
+from illume_amd._abi import render_params
+
+pytestmark = pytest.mark.gpu
+
+TAIL = 1 << 18
+SCENES = {"cornell": S.cornell, "tiny": S.tiny_mesh_scene, "gold": lambda: S.gold_spheres(n=20),
+          "medium": lambda: S.subsurface(n=12, env_size=(64, 32))}
+
+
+@pytest.fixture(scope="module")
+def pair():
+    with illume_amd.Context(0, extend_mode=3) as a, illume_amd.Context(0) as b:
+        yield a, b
+
+
+# one path; a wave's four, 64 and 65; every wave of the launch with 4 and 5 paths; the limit itself, one row
+# above it (the queue crosses the limit after some depths) and a queue that stays above it
+@pytest.mark.parametrize("name,w,h,spp,depth", [
+    ("tiny", 1, 1, 1, 12), ("tiny", 4, 1, 1, 12), ("cornell", 64, 1, 1, 8), ("tiny", 13, 5, 1, 1),
+    ("medium", 160, 128, 1, 45), ("gold", 160, 128, 1, 16), ("medium", 5121, 5, 1, 45),
+    ("tiny", 512, 512, 1, 12), ("tiny", 512, 513, 1, 12), ("cornell", 512, 513, 1, 8), ("medium", 333, 251, 7, 45),
+    ("cornell", 700, 700, 3, 3)])
+@pytest.mark.parametrize("layout,tri", [("fp32", "mt"), ("quant8", "mt"), ("fp32", "watertight")])
+def test_short_queues_match_the_per_depth_kernels(name, w, h, spp, depth, layout, tri):
+    spec, st = SCENES[name]()
+    p = render_params(**dict(st, width=w, height=h, spp=spp, max_depth=depth))
+    out = []
+    for mode in (3, 0):
+        with illume_amd.Context(0, extend_mode=mode, bvh_layout=layout, tri_test=tri, paths_in_flight=1 << 21) as c:
+            s = c.scene(spec)
+            out.append(c.render(s, p))
+            if mode == 0:
+                out.append(c.render(s, p))          # the captured graph again
+                out.append(c.render_noalloc(s, p))
+            s.free()
+    ref = out[0]
+    for a, px, info in out[1:]:
+        assert np.array_equal(a, ref[0], equal_nan=True)
+        assert np.array_equal(px, ref[1])
+        assert info["segments"] == ref[2]["segments"]
+
+
+def test_short_queues_of_several_scenes_match(pair):
+    """A chunk of several scenes, below the limit and crossing it, served and batched."""
+    reqs = [("cornell", 64, 48, 3), ("tiny", 50, 33, 5), ("gold", 40, 40, 2), ("medium", 31, 57, 3), ("tiny", 400, 300, 3)]
+    res = []
+    for c in pair:
+        sc = {k: c.scene(SCENES[k]()[0]) for k in SCENES}
+        ps = [render_params(**dict(SCENES[k]()[1], width=w, height=h, spp=n)) for k, w, h, n in reqs]
+        small, i0 = c.render_batch([sc[r[0]] for r in reqs[:4]], ps[:4])
+        big, i1 = c.render_batch([sc[r[0]] for r in reqs], ps)
+        hs = [c.submit(sc[r[0]], p) for r, p in zip(reqs, ps)]
+        served = []
+        for h in hs:
+            h.wait(60000)
+            served.append(h.result())
+            h.free()
+        for s in sc.values():
+            s.free()
+        res.append((small + big + served, i0["segments"], i1["segments"]))
+    for (a, ap), (b, bp) in zip(res[0][0], res[1][0]):
+        assert np.array_equal(a, b, equal_nan=True) and np.array_equal(ap, bp)
+    assert res[0][1:] == res[1][1:]
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 65, 5120 * 16 + 1, TAIL, TAIL + 1])
+def test_closest_hits_of_short_queues_match(pair, n):
+    rng = np.random.default_rng(n)
+    rays = np.concatenate([rng.uniform(-3, 3, (n, 3)), rng.normal(size=(n, 3))], 1)
+    rays[::7, 3] = 0.0                               # axis-parallel planes
+    rays[::11, 4:] = 0.0
+    rays[:, 3:] /= np.maximum(np.linalg.norm(rays[:, 3:], axis=1, keepdims=True), 1e-9)
+    spec, _ = S.tiny_mesh_scene(n=9)
+    out = []
+    for c in pair:
+        s = c.scene(spec)
+        out.append(c.closest_hit(s, rays))
+        s.free()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
