@@ -29,6 +29,7 @@ struct ilm_scene {
     std::vector<float> inst_mats;   /* 48 per instance: mat, inv, inverse-transpose */
     int num_instances = 0;
     int64_t mesh_tris = 0;
+    int64_t inst_tris = 0;      /* triangles over all instances */
     int stack_bound_fp32 = 0;
     int stack_bound_q = 0;
     int stack_bound_f = 0;      /* quad walk over FNodes */

@@ -291,6 +291,7 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
         m4_rows(inv, di.inv);
         m4_rows(tinv, di.tinv);
         di.mesh = d->instances[i].mesh;
+        s->inst_tris += d->meshes[di.mesh].num_triangles;
         di.material = d->instances[i].material;
         di.nodes = dmeshes[di.mesh].nodes;
         di.qnodes = dmeshes[di.mesh].qnodes;
@@ -819,6 +820,20 @@ static void chunk_choices(const ilm_ctx* ctx, uint32_t total_paths, bool quad_fi
     P.tail_only = (int64_t)total_paths <= (int64_t)P.quad_max ? 1 : 0;
 }
 
+/* Whether a request's camera rays are traced as packets by default. A packet visits the union of
+ * its 64 rays' walks, and one wave carries it to its end, so it pays while the 64 / sgroup pixels
+ * it covers show few triangles; the scene's triangles per image pixel stand for that. First-depth
+ * time as packets / per lane, 8-bit nodes (FP32 nodes within 0.1, except where given), by
+ * triangles in the footprint: 100k triangles at 1920x1080 0.90 (0.8, 4 samples), 1.01 (1.6, 2),
+ * 1.10 (3.2, 1); at 640x480 1.03 (2.6, 8), 1.06 (5, 4), 1.29 (10, 2; FP32 1.12), 1.57 (21, 1);
+ * 11 small meshes 0.81 (2.4, 4), 0.97 (4.8, 2), 1.23 (9.6, 1); 525k triangles 0.97 (3, 16), 1.04
+ * (6, 8), 1.07 (12, 4), 1.66 (24, 2); 12 instances of 722k 0.99 (19, 32; FP32 0.87), 1.27 (37,
+ * 16), 1.77 (150, 4), 4.2 (600, 1). */
+#define ILM_PACKET_MAX_TRIS 20
+static bool packet_pays(const ilm_scene* s, const ilm_render_params& p, uint32_t sgroup) {
+    return sgroup >= 2 && (double)s->inst_tris * 64.0 <= ILM_PACKET_MAX_TRIS * (double)sgroup * p.width * p.height;
+}
+
 /* Stage a chunk descriptor: pinned ring slot -> the device DChunk dst (ordered on stream s). */
 static int stage_chunk(ilm_ctx* ctx, const DChunk& hc, DChunk* dst, hipStream_t s) {
     int slot = ctx->ring_pos++ % ILM_RING;
@@ -929,9 +944,14 @@ static int launch_chunk(ilm_ctx* ctx, const DChunk& hc, const std::vector<Job*>&
     const bool uni = chunk_uni_scene(hc);
     P.uni_scene = uni ? 1 : 0;
     chunk_choices(ctx, hc.total_paths, jobs_fit_quad(jobs), P);
+    if (ctx->opts.camera_packets == 0)
+        for (int w = 0; w < hc.n_work && P.packet0; w++) {
+            const Job* j = jobs[hc.work[w].req];
+            P.packet0 = packet_pays(j->scene, j->p, hc.work[w].sgroup) ? 1 : 0;
+        }
     const int D = hc.depth_steps;
     const bool graphs = ctx->opts.use_graphs && !prof && !ctx->opts.count_tests;
-    if (graphs) rc = run_graph(ctx, 2 * (32 * D + 16 * (P.quad_max > 0) + 8 * P.tail_only + 4 * k + (uni ? 2 : 0) + (ovf ? 1 : 0)), q, P, D, false);
+    if (graphs) rc = run_graph(ctx, 2 * (64 * D + 32 * P.packet0 + 16 * (P.quad_max > 0) + 8 * P.tail_only + 4 * k + (uni ? 2 : 0) + (ovf ? 1 : 0)), q, P, D, false);
     else rc = enqueue_depths(ctx, q, P, D, prof);
     if (rc) return rc;
     if (ctx->npipes == 2) {
@@ -1431,6 +1451,7 @@ int ilm_render_noalloc(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* 
         P.use_ovf = spill ? 1 : 0;
         P.uni_scene = 1;
         chunk_choices(ctx, hc.total_paths, scene_fits_quad(scene), P);
+        if (ctx->opts.camera_packets == 0) P.packet0 = packet_pays(scene, *params, hc.work[0].sgroup) ? 1 : 0;
         rc = enqueue_pipeline(ctx, q, P, hc.depth_steps, nullptr);
         if (rc) return rc;
         chunks++;

@@ -824,8 +824,15 @@ template <int T, int Q, int C, int O>
 static void launch_extend(const KParams& P, int depth, int* ovf, int grid, hipStream_t s) {
     if (P.extend_mode == ILM_EXTEND_STEP_REFILL && P.cam0 && P.packet0 && depth == 0)
         ILM_LAUNCH((k_extend_packet<T, Q, C>), dim3(grid), dim3(EXT_BLOCK), 0, s, P, depth);
-    else if (P.extend_mode == ILM_EXTEND_STEP_REFILL && P.cam0 && depth == 0)
+    else if (P.extend_mode == ILM_EXTEND_STEP_REFILL && P.cam0 && depth == 0) {
+        if constexpr (C == 0) {
+            if (P.uni_scene) {
+                ILM_LAUNCH((k_extend_pers<T, Q, 0, O, 1, 1>), dim3(grid), dim3(EXT_BLOCK), 0, s, P, depth, ovf);
+                return;
+            }
+        }
         ILM_LAUNCH((k_extend_pers<T, Q, C, O, 1, 0>), dim3(grid), dim3(EXT_BLOCK), 0, s, P, depth, ovf);
+    }
     else if (P.extend_mode == ILM_EXTEND_STEP_REFILL) {
         if constexpr (C == 0) {
             if (P.uni_scene) {

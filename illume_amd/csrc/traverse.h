@@ -764,7 +764,7 @@ __device__ inline uint32_t pool_fetch(uint32_t count, uint32_t fetch) {
 }
 
 /* First depth with per-step refill: each wave reserves consecutive path ids (P.ext_fetch per
- * queue atomic, shrinking to 64 as the queue drains, as in k_extend), and traces them 64 at a
+ * queue atomic, less for a queue that is short for the grid or drains), and traces them 64 at a
  * time: forms their camera rays (camera_ray) and walks one packet per distinct scene among them.
  * Every path id of the chunk passes through here once, so the kernel also clears the per-path
  * results (the chunk needs no separate clear). */
@@ -1309,6 +1309,8 @@ __global__ EXT_BOUNDS void k_extend_pers(KParams P, int depth, int* ovf_base) {
     if (UNI) U = uscene_load<QUANT>(Su);
     const uint32_t refill_min = (uint32_t)P.refill_min;
     const uint32_t leaf_pct = (uint32_t)P.leaf_pct;
+    CamSrc cs;
+    const bool cu = CAM && UNI && camsrc_load(P, cs);
     uint32_t ridx = NO_RAY;
     uint32_t pool, pool_end;
     pool_first(count, fetch, pool, pool_end);
@@ -1336,7 +1338,8 @@ __global__ EXT_BOUNDS void k_extend_pers(KParams P, int depth, int* ovf_base) {
                         /* camera rays start outside every medium: no free-flight cap */
                         float4 o4, d4;
                         uint2 rg;
-                        camera_ray(P, r, o4, d4, rg);
+                        if (UNI && cu) camera_ray_u(camu_fetch(cs), r, o4, d4, rg);
+                        else camera_ray(P, r, o4, d4, rg);
                         const GLOBAL DScene* S = UNI ? Su : gp(reqs[f2u(o4.w) >> 16].scene);
                         pstep_init<QUANT, OVF, UNI, COUNT>(T, B, st, S, U, mk3(o4.x, o4.y, o4.z),
                                                            mk3(d4.x, d4.y, d4.z), ILM_FLT_MAX, &tc);

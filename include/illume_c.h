@@ -230,8 +230,9 @@ typedef struct ilm_opts {
      * ones. Results are identical either way. */
     int32_t sched_fair;
     /* first depth with per-step refill: trace each wave's 64 camera rays as one packet (one
-     * traversal for the wave, every lane testing its own ray; 0 = default: on, 1 = on, 2 = off,
-     * each lane walking alone). Results are identical either way. */
+     * traversal for the wave, every lane testing its own ray; 0 = default: where a packet's
+     * pixels show few triangles, 1 = on, 2 = off, each lane walking alone). Results are
+     * identical either way. */
     int32_t camera_packets;
     /* chunk pipelines (1 or 2; 0 = 2): consecutive chunks alternate between two sets of path
      * buffers on two streams, so a chunk's last, short launches run beside the next chunk's

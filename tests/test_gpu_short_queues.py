@@ -85,3 +85,21 @@ def test_closest_hits_of_short_queues_match(pair, n):
         s.free()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("layout", ["fp32", "quant8"])
+@pytest.mark.parametrize("w,h,spp", [(1024, 512, 1), (1024, 512, 2), (333, 331, 8), (96, 64, 64), (700, 701, 3)])
+def test_camera_rays_per_lane_and_as_packets_match(w, h, spp, layout):
+    """The default choice between packets and lanes for the first depth, and both by name, over
+    queues of few and many rays per wave (whole and split, ragged, one to 64 samples a pixel)."""
+    spec, st = SCENES["tiny"]()
+    p = render_params(**dict(st, width=w, height=h, spp=spp, max_depth=3))
+    out = []
+    for packets in (0, 1, 2):
+        with illume_amd.Context(0, extend_mode=3, camera_packets=packets, bvh_layout=layout) as c:
+            s = c.scene(spec)
+            out.append(c.render(s, p))
+            s.free()
+    for a, px, info in out[1:]:
+        assert np.array_equal(a, out[0][0], equal_nan=True) and np.array_equal(px, out[0][1])
+        assert info["segments"] == out[0][2]["segments"]
