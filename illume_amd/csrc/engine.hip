@@ -619,6 +619,7 @@ int ilm_open(int device, const ilm_opts* opts, ilm_ctx** out) {
     HIPTRY(ctx, hipHostMalloc((void**)&ctx->h_u64, 4 * sizeof(unsigned long long), hipHostMallocDefault));
     HIPTRY(ctx, hipHostMalloc((void**)&ctx->h_seg_ring, ILM_RING * sizeof(unsigned long long), hipHostMallocDefault));
     for (int i = 0; i < 2; i++) HIPTRY(ctx, hipEventCreate(&ctx->na_ev[i]));
+    for (int i = 0; i < 2; i++) HIPTRY(ctx, hipEventCreate(&ctx->rend_ev[i]));
     HIPTRY(ctx, noalloc_scratch_of(device, &ctx->noalloc_scratch));
     size_t free_b = 0, total_b = 0;
     HIPTRY(ctx, hipMemGetInfo(&free_b, &total_b));
@@ -628,6 +629,7 @@ int ilm_open(int device, const ilm_opts* opts, ilm_ctx** out) {
 }
 
 static void server_stop(ilm_ctx* ctx);
+static void stage_free(ilm_ctx* ctx, Staging* g);
 
 static void ctx_destroy(ilm_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
@@ -638,6 +640,8 @@ static void ctx_destroy(ilm_ctx* ctx) {
     dfree(ctx->device, ctx->ovf);
     for (auto& kv : ctx->bufs.free) dfree(ctx->device, kv.second);
     ctx->bufs.free.clear();
+    for (Staging* g : ctx->stages.free) stage_free(ctx, g);
+    ctx->stages.free.clear();
     for (void* p : ctx->allocs) dfree(ctx->device, p);
     dfree(ctx->device, ctx->seg_count);
     for (int i = 0; i < ILM_RING; i++) {
@@ -648,6 +652,7 @@ static void ctx_destroy(ilm_ctx* ctx) {
     if (ctx->h_seg_ring) (void)hipHostFree(ctx->h_seg_ring);
     for (int i = 0; i < 2; i++) {
         if (ctx->na_ev[i]) (void)hipEventDestroy(ctx->na_ev[i]);
+        if (ctx->rend_ev[i]) (void)hipEventDestroy(ctx->rend_ev[i]);
         if (ctx->acc_ev[i]) (void)hipEventDestroy(ctx->acc_ev[i]);
     }
     if (ctx->fill_ev) (void)hipEventDestroy(ctx->fill_ev);
@@ -989,22 +994,25 @@ static void job_fill_req(Job* j) {
     j->next_px = 0;
 }
 
-static int job_prepare(ilm_ctx* ctx, Job* j) {
+/* begin: the first request of a plain or batched render, whose clear also starts the render's
+ * counters (k_begin). */
+static int job_prepare(ilm_ctx* ctx, Job* j, bool begin) {
     const ilm_render_params& p = j->p;
     const int64_t wh = (int64_t)p.width * p.height;
-    const size_t ab = 2 * wh * sizeof(float4), pb = wh * sizeof(ilm_pixel);
+    const size_t ab = 2 * wh * sizeof(float4), pb = wh * sizeof(uint32_t);
     j->pool = &ctx->bufs;
     j->d_accum = (float4*)ctx->bufs.take(ab, &j->accum_cap);
     if (!j->d_accum) {
         HIPTRY(ctx, hipMalloc((void**)&j->d_accum, ab));
         j->accum_cap = ab;
     }
-    j->d_px = (ilm_pixel*)ctx->bufs.take(pb, &j->px_cap);
+    j->d_px = (uint32_t*)ctx->bufs.take(pb, &j->px_cap);
     if (!j->d_px) {
         HIPTRY(ctx, hipMalloc((void**)&j->d_px, pb));
         j->px_cap = pb;
     }
-    HIPTRY(ctx, ilm_k_fill_zero4(j->d_accum, 2 * wh, ctx->stream));
+    if (begin) HIPTRY(ctx, ilm_k_begin(j->d_accum, 2 * wh, ctx->d_seg_total, ctx->d_trav, ctx->h_u64, ctx->stream));
+    else HIPTRY(ctx, ilm_k_fill_zero4(j->d_accum, 2 * wh, ctx->stream));
     HIPTRY(ctx, hipEventRecord(ctx->fill_ev, ctx->stream));
     job_fill_req(j);
     return ILM_OK;
@@ -1169,20 +1177,209 @@ static int check_scene_stack(ilm_ctx* ctx, const ilm_scene* s) {
     return ILM_OK;
 }
 
-static void accum4_to_rgb(const std::vector<float4>& a4, float* rgb, int64_t n) {
-    for (int64_t i = 0; i < n; i++) { rgb[3 * i] = a4[i].x; rgb[3 * i + 1] = a4[i].y; rgb[3 * i + 2] = a4[i].z; }
+/* ======================= results ======================= */
+
+/* A result of n pixels in staging memory: packed RGB sums, then pixel words (k_send), each with
+ * room for n rounded up to four. */
+static int64_t stage_round(int64_t n) { return (n + 3) & ~(int64_t)3; }
+static size_t stage_bytes(int64_t n) { return (size_t)stage_round(n) * 16; }
+
+static void stage_free(ilm_ctx* ctx, Staging* g) {
+    if (!g) return;
+    {
+        std::lock_guard<std::mutex> cap(capture_mu(ctx->device));
+        if (g->p) (void)hipHostFree(g->p);
+    }
+    for (hipEvent_t e : g->ev)
+        if (e) (void)hipEventDestroy(e);
+    delete g;
+}
+static Staging* stage_take(ilm_ctx* ctx, size_t bytes) {
+    {
+        std::lock_guard<std::mutex> lk(ctx->stages.mu);
+        std::vector<Staging*>& f = ctx->stages.free;
+        size_t best = f.size();
+        for (size_t k = 0; k < f.size(); k++)
+            if (f[k]->cap >= bytes && f[k]->cap / 2 <= bytes + (1 << 20) && (best == f.size() || f[k]->cap < f[best]->cap)) best = k;
+        if (best < f.size()) {
+            Staging* g = f[best];
+            f.erase(f.begin() + best);
+            ctx->stages.bytes -= g->cap;
+            return g;
+        }
+    }
+    std::unique_ptr<Staging> g(new (std::nothrow) Staging());
+    if (!g) return nullptr;
+    hipError_t e;
+    {
+        std::lock_guard<std::mutex> cap(capture_mu(ctx->device));
+        e = hipHostMalloc(&g->p, bytes, hipHostMallocDefault);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    g->cap = bytes;
+    return g.release();
+}
+static void stage_give(ilm_ctx* ctx, Staging* g) {
+    if (!g) return;
+    {
+        std::lock_guard<std::mutex> lk(ctx->stages.mu);
+        if (ctx->stages.bytes + g->cap <= ctx->stages.cap) {
+            ctx->stages.free.push_back(g);
+            ctx->stages.bytes += g->cap;
+            return;
+        }
+    }
+    stage_free(ctx, g);
+}
+
+/* A run of one result's pixels on its way to the caller: sent to the staging buffer's bytes at
+ * off by one k_send, complete once the event is. */
+struct Piece {
+    const float4* d_sums;
+    const uint32_t* d_px;
+    int64_t n;
+    size_t off;
+    hipEvent_t ev;          /* null: already complete */
+    float* rgb;             /* the caller's arrays at the piece's first pixel; either may be null */
+    ilm_pixel* px;
+};
+static void piece_unpack(const Staging* g, const Piece& p, int64_t lo, int64_t hi) {
+    const float* rgb = (const float*)((const char*)g->p + p.off);
+    const uint32_t* px = (const uint32_t*)(rgb + 3 * stage_round(p.n));
+    if (p.rgb) std::memcpy(p.rgb + 3 * lo, rgb + 3 * lo, (size_t)(hi - lo) * 3 * sizeof(float));
+    if (p.px)
+        for (int64_t i = lo; i < hi; i++) {
+            const uint32_t v = px[i];
+            p.px[i].r = v & 255u;
+            p.px[i].g = (v >> 8) & 255u;
+            p.px[i].b = (v >> 16) & 255u;
+        }
+}
+
+/* Unpack the pieces into the caller's arrays as they arrive. The caller's memory is usually fresh,
+ * so this is bound by its page faults and stores: 1920x1080 takes one thread 4.9 to 12 ms, two
+ * 2.7, four 1.5, eight 1.1. Small results stay on the calling thread (a thread costs some 20 us). */
+#define ILM_UNPACK_PX 16384
+static int unpack_pieces(ilm_ctx* ctx, const Staging* g, const std::vector<Piece>& pieces) {
+    struct Item { int piece; int64_t lo, hi; };
+    std::vector<Item> items;
+    for (size_t k = 0; k < pieces.size(); k++)
+        for (int64_t lo = 0; lo < pieces[k].n; lo += ILM_UNPACK_PX)
+            items.push_back({(int)k, lo, std::min<int64_t>(pieces[k].n, lo + ILM_UNPACK_PX)});
+    std::atomic<size_t> next{0};
+    std::atomic<int> bad{(int)hipSuccess};
+    auto work = [&] {
+        int seen = -1;
+        for (size_t i; (i = next.fetch_add(1)) < items.size();) {
+            const Item& it = items[i];
+            if (it.piece > seen) {
+                if (pieces[it.piece].ev) {
+                    const hipError_t e = hipEventSynchronize(pieces[it.piece].ev);
+                    if (e != hipSuccess) { bad.store((int)e); return; }
+                }
+                seen = it.piece;
+            }
+            piece_unpack(g, pieces[it.piece], it.lo, it.hi);
+        }
+    };
+    const unsigned hw = std::thread::hardware_concurrency();
+    const size_t helpers = std::min<size_t>({(size_t)7, items.size() / 2, (size_t)(hw / 2)});
+    std::vector<std::thread> th;
+    try {
+        th.reserve(helpers);
+        for (size_t k = 0; k < helpers; k++) th.emplace_back(work);
+    } catch (...) {   /* no more threads: those there are, and this one, do the rest */
+    }
+    work();
+    for (std::thread& t : th) t.join();
+    const hipError_t e = (hipError_t)bad.load();
+    if (e != hipSuccess) return fail(ctx, ILM_E_DEVICE, std::string("result transfer: ") + hipGetErrorString(e));
+    return ILM_OK;
+}
+
+/* Results of a plain or batched call, sent and unpacked in rounds of at most ILM_STAGE_ROUND bytes
+ * of staging memory. The first round is queued on the render's stream right behind it, the others
+ * (large batches) on the copy stream. */
+#define ILM_STAGE_ROUND ((size_t)64 << 20)
+#define ILM_PIECE_PX (1 << 18)
+struct Delivery {
+    std::vector<Piece> all;     /* every piece of the call */
+    size_t done = 0;            /* pieces unpacked */
+    std::vector<Piece> round;   /* the round in flight */
+    Staging* g = nullptr;
+};
+static void delivery_plan(Delivery& d, Job* j, float* rgb, ilm_pixel* px) {
+    if (!rgb && !px) return;
+    const int64_t wh = (int64_t)j->p.width * j->p.height;
+    for (int64_t p0 = 0; p0 < wh; p0 += ILM_PIECE_PX) {
+        Piece p = {j->d_accum + p0, j->d_px + p0, std::min<int64_t>(wh - p0, ILM_PIECE_PX), 0, nullptr,
+                   rgb ? rgb + 3 * p0 : nullptr, px ? px + p0 : nullptr};
+        d.all.push_back(p);
+    }
+}
+static int delivery_send(ilm_ctx* ctx, Delivery& d, hipStream_t s) {
+    d.round.clear();
+    size_t bytes = 0;
+    while (d.done + d.round.size() < d.all.size() && d.round.size() < ILM_STAGE_EVENTS) {
+        Piece p = d.all[d.done + d.round.size()];
+        const size_t b = stage_bytes(p.n);
+        if (!d.round.empty() && bytes + b > ILM_STAGE_ROUND) break;
+        p.off = bytes;
+        bytes += b;
+        d.round.push_back(p);
+    }
+    if (d.round.empty()) return ILM_OK;
+    if (!d.g || d.g->cap < bytes) {
+        stage_give(ctx, d.g);
+        d.g = stage_take(ctx, bytes);
+        if (!d.g) return fail(ctx, ILM_E_NOMEM, "pinned result buffer");
+    }
+    for (size_t k = 0; k < d.round.size(); k++) {
+        Piece& p = d.round[k];
+        float* rgb = (float*)((char*)d.g->p + p.off);
+        uint32_t* px = (uint32_t*)(rgb + 3 * stage_round(p.n));
+        HIPTRY(ctx, ilm_k_send(p.d_sums, p.d_px, p.rgb ? rgb : nullptr, p.px ? px : nullptr, (int)p.n, s));
+        if (!d.g->ev[k]) HIPTRY(ctx, hipEventCreateWithFlags(&d.g->ev[k], hipEventDisableTiming));
+        HIPTRY(ctx, hipEventRecord(d.g->ev[k], s));
+        p.ev = d.g->ev[k];
+    }
+    return ILM_OK;
+}
+/* Unpack the round in flight, then send and unpack the rest. */
+static int delivery_finish(ilm_ctx* ctx, Delivery& d) {
+    int rc = ILM_OK;
+    while (!rc && !d.round.empty()) {
+        rc = unpack_pieces(ctx, d.g, d.round);
+        d.done += d.round.size();
+        if (!rc) rc = delivery_send(ctx, d, ctx->copy_stream);
+    }
+    return rc;
+}
+/* Give the staging buffer back; nothing may still be writing to it. */
+static void delivery_end(ilm_ctx* ctx, Delivery& d, bool failed) {
+    if (failed) {
+        (void)hipStreamSynchronize(ctx->stream);
+        (void)hipStreamSynchronize(ctx->copy_stream);
+    }
+    stage_give(ctx, d.g);
+    d.g = nullptr;
 }
 
 /* a lone request of at least this many paths is rendered as two chunks (run_jobs_sync) */
 #define ILM_SPLIT_MIN_PATHS (1LL << 22)
 #define ILM_SPLIT_MIN_DEPTH 24
 
-/* Run jobs to completion on the calling thread (plain and batched forms). */
-static int run_jobs_sync(ilm_ctx* ctx, std::vector<Job*>& jobs, ilm_render_info* info) {
+/* Run jobs on the calling thread (plain and batched forms). On return every kernel of the renders
+ * is done and dl's first round of results is on its way. */
+static int run_jobs_sync(ilm_ctx* ctx, std::vector<Job*>& jobs, float* const* accum_rgb, ilm_pixel* const* out, Delivery& dl,
+                         ilm_render_info* info) {
     std::lock_guard<std::mutex> dev(ctx->dev_mu);
     HIPTRY(ctx, hipSetDevice(ctx->device));
     for (Job* j : jobs) {
-        int rc = job_prepare(ctx, j);
+        int rc = job_prepare(ctx, j, j == jobs[0]);
         if (rc) return rc;
         /* pass i of the render seeds wang_hash(first_sample + i) */
         j->next_pass = 0;
@@ -1205,12 +1402,7 @@ static int run_jobs_sync(ilm_ctx* ctx, std::vector<Job*>& jobs, ilm_render_info*
             j->split_npx = (((wh + 1) / 2) + 63) & ~(int64_t)63;
     }
     ProfileSink prof;
-    hipEvent_t e0, e1;
-    HIPTRY(ctx, hipEventCreate(&e0));
-    HIPTRY(ctx, hipEventCreate(&e1));
-    /* the segment counter is cumulative; read it before and after */
-    HIPTRY(ctx, hipMemcpyAsync(ctx->h_u64 + 3, ctx->d_seg_total, sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx->stream));
-    HIPTRY(ctx, hipMemsetAsync(ctx->d_trav, 0, 2 * sizeof(unsigned long long), ctx->stream));
+    const hipEvent_t e0 = ctx->rend_ev[0], e1 = ctx->rend_ev[1];
     HIPTRY(ctx, hipEventRecord(e0, ctx->stream));
     if (ctx->stream2) HIPTRY(ctx, hipStreamWaitEvent(ctx->stream2, e0, 0));
     DChunk* hc = new DChunk();
@@ -1231,18 +1423,20 @@ static int run_jobs_sync(ilm_ctx* ctx, std::vector<Job*>& jobs, ilm_render_info*
     /* the latest accumulation follows every earlier one, and each chunk's depths precede its
      * accumulation on its stream */
     if (chunks && ctx->last_pipe != 0) HIPTRY(ctx, hipStreamWaitEvent(ctx->stream, ctx->acc_ev[ctx->last_pipe], 0));
-    for (Job* j : jobs) {
+    for (size_t k = 0; k < jobs.size(); k++) {
+        Job* j = jobs[k];
         const int64_t wh = (int64_t)j->p.width * j->p.height;
-        HIPTRY(ctx, ilm_k_tonemap(j->d_accum, j->d_px, (int)wh, j->p.spp, j->p.tonemap, ctx->stream));
+        /* the last one leaves the counters (the segment counter is cumulative: k_begin's value off) */
+        HIPTRY(ctx, ilm_k_tonemap8(j->d_accum, j->d_px, (int)wh, j->p.spp, j->p.tonemap, ctx->d_seg_total, ctx->d_trav,
+                                   k + 1 == jobs.size() ? ctx->h_u64 : nullptr, ctx->stream));
     }
     HIPTRY(ctx, hipEventRecord(e1, ctx->stream));   /* device_ms: every kernel of the render, tonemap included */
-    HIPTRY(ctx, hipMemcpyAsync(ctx->h_u64, ctx->d_seg_total, sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx->stream));
-    HIPTRY(ctx, hipMemcpyAsync(ctx->h_u64 + 1, ctx->d_trav, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx->stream));
-    HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
+    for (size_t k = 0; k < jobs.size(); k++) delivery_plan(dl, jobs[k], accum_rgb ? accum_rgb[k] : nullptr, out ? out[k] : nullptr);
+    int rc = delivery_send(ctx, dl, ctx->stream);
+    if (rc) return rc;
+    HIPTRY(ctx, hipEventSynchronize(e1));
     float ms = 0.0f;
     HIPTRY(ctx, hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
     double ext_ms = 0.0;
     for (auto& pr : prof.ev) {
         float m = 0.0f;
@@ -1270,17 +1464,6 @@ static int run_jobs_sync(ilm_ctx* ctx, std::vector<Job*>& jobs, ilm_render_info*
     return ILM_OK;
 }
 
-static int copy_job_outputs(ilm_ctx* ctx, Job* j, float* accum_rgb, ilm_pixel* out) {
-    const int64_t wh = (int64_t)j->p.width * j->p.height;
-    if (accum_rgb) {
-        std::vector<float4> a4(wh);
-        HIPTRY(ctx, copy_sync(ctx, a4.data(), j->d_accum, wh * sizeof(float4), hipMemcpyDeviceToHost));
-        accum4_to_rgb(a4, accum_rgb, wh);
-    }
-    if (out) HIPTRY(ctx, copy_sync(ctx, out, j->d_px, wh * sizeof(ilm_pixel), hipMemcpyDeviceToHost));
-    return ILM_OK;
-}
-
 int ilm_render(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params, float* accum_rgb, ilm_pixel* out,
                ilm_render_info* info) {
     if (!ctx || !scene) return fail(ctx, ILM_E_INVALID, "null context or scene");
@@ -1292,8 +1475,10 @@ int ilm_render(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params, 
     j.p = *params;
     std::vector<Job*> jobs = {&j};
     if (info) std::memset(info, 0, sizeof(*info));
-    rc = run_jobs_sync(ctx, jobs, info);
-    if (!rc) rc = copy_job_outputs(ctx, &j, accum_rgb, out);
+    Delivery dl;
+    rc = run_jobs_sync(ctx, jobs, &accum_rgb, &out, dl, info);
+    if (!rc) rc = delivery_finish(ctx, dl);
+    delivery_end(ctx, dl, rc != ILM_OK);
     job_release_device(&j);
     return rc;
 }
@@ -1320,7 +1505,10 @@ int ilm_render_batch(ilm_ctx* ctx, int32_t n, ilm_scene* const* scenes, const il
         std::vector<Job*> grp(jobs.begin() + g, jobs.begin() + std::min(n, g + ILM_MAX_JOBS));
         ilm_render_info gi;
         std::memset(&gi, 0, sizeof(gi));
-        rc = run_jobs_sync(ctx, grp, &gi);
+        Delivery dl;
+        rc = run_jobs_sync(ctx, grp, accum_rgb ? accum_rgb + g : nullptr, out ? out + g : nullptr, dl, &gi);
+        if (!rc) rc = delivery_finish(ctx, dl);
+        delivery_end(ctx, dl, rc != ILM_OK);
         if (info) {
             info->segments += gi.segments;
             info->device_ms += gi.device_ms;
@@ -1330,10 +1518,6 @@ int ilm_render_batch(ilm_ctx* ctx, int32_t n, ilm_scene* const* scenes, const il
             info->paths_per_chunk = std::max(info->paths_per_chunk, gi.paths_per_chunk);
             info->box_tests += gi.box_tests;
             info->tri_tests += gi.tri_tests;
-        }
-        for (size_t k = 0; k < grp.size() && !rc; k++) {
-            int i = g + (int)k;
-            rc = copy_job_outputs(ctx, grp[k], accum_rgb ? accum_rgb[i] : nullptr, out ? out[i] : nullptr);
         }
         for (Job* j : grp) job_release_device(j);
     }
@@ -1679,10 +1863,11 @@ static void server_loop(ilm_ctx* ctx) {
                 for (Job* j : in_chunk) {
                     if (!job_has_work(j)) {
                         const int64_t wh = (int64_t)j->p.width * j->p.height;
-                        if (ilm_k_tonemap(j->d_accum, j->d_px, (int)wh, j->p.spp, j->p.tonemap, q.stream) != hipSuccess)
+                        float* rgb = (float*)j->stage->p;
+                        if (ilm_k_tonemap8(j->d_accum, j->d_px, (int)wh, j->p.spp, j->p.tonemap, nullptr, nullptr, nullptr,
+                                           q.stream) != hipSuccess ||
+                            ilm_k_send(j->d_accum, j->d_px, rgb, (uint32_t*)(rgb + 3 * stage_round(wh)), (int)wh, q.stream) != hipSuccess)
                             j->failed = true;
-                        (void)hipMemcpyAsync(j->h_accum, j->d_accum, wh * sizeof(float4), hipMemcpyDeviceToHost, q.stream);
-                        (void)hipMemcpyAsync(j->h_px, j->d_px, wh * sizeof(ilm_pixel), hipMemcpyDeviceToHost, q.stream);
                         f.finishing.push_back(j);
                     }
                 }
@@ -1755,7 +1940,7 @@ static void admit_prepare(ilm_ctx* ctx, std::vector<Job*>& picked) {
         int rc;
         {
             std::lock_guard<std::mutex> dev(ctx->dev_mu);
-            rc = job_prepare(ctx, j);
+            rc = job_prepare(ctx, j, false);
             if (rc != ILM_OK) job_release_device(j);
         }
         std::lock_guard<std::mutex> lk(ctx->sched_mu);
@@ -1803,15 +1988,10 @@ int ilm_submit(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params, 
     j->scene = scene;
     j->p = *params;
     j->bytes = wh * (2 * (int64_t)sizeof(float4) + (int64_t)sizeof(ilm_pixel));
-    j->device = ctx->device;
-    bool pinned;
-    {
-        std::lock_guard<std::mutex> cap(capture_mu(ctx->device));
-        pinned = hipHostMalloc((void**)&j->h_accum, wh * sizeof(float4), hipHostMallocDefault) == hipSuccess &&
-                 hipHostMalloc((void**)&j->h_px, wh * sizeof(ilm_pixel), hipHostMallocDefault) == hipSuccess;
-    }
-    if (!pinned) {
-        delete j;   /* ~Job frees whichever buffer was allocated */
+    j->ctx = ctx;
+    j->stage = stage_take(ctx, stage_bytes(wh));
+    if (!j->stage) {
+        delete j;
         return fail(ctx, ILM_E_NOMEM, "pinned result buffers");
     }
     {
@@ -1874,14 +2054,8 @@ int ilm_result(ilm_req* r, float* accum_rgb, ilm_pixel* out) {
     Job* j = r->job;
     if (j->state.load() != ILM_REQ_DONE) return fail(r->ctx, ILM_E_STATE, "request not done");
     const int64_t wh = (int64_t)j->p.width * j->p.height;
-    if (accum_rgb)
-        for (int64_t i = 0; i < wh; i++) {
-            accum_rgb[3 * i] = j->h_accum[i].x;
-            accum_rgb[3 * i + 1] = j->h_accum[i].y;
-            accum_rgb[3 * i + 2] = j->h_accum[i].z;
-        }
-    if (out) std::memcpy(out, j->h_px, wh * sizeof(ilm_pixel));
-    return ILM_OK;
+    const std::vector<Piece> whole = {{nullptr, nullptr, wh, 0, nullptr, accum_rgb, out}};
+    return unpack_pieces(r->ctx, j->stage, whole);
 }
 
 int ilm_cancel(ilm_req* r) {
@@ -1911,10 +2085,7 @@ void ilm_req_free(ilm_req* r) {
 }
 
 Job::~Job() {
-    if (!h_accum && !h_px) return;
-    std::lock_guard<std::mutex> lk(capture_mu(device));
-    if (h_accum) (void)hipHostFree(h_accum);
-    if (h_px) (void)hipHostFree(h_px);
+    if (stage) stage_give(ctx, stage);
 }
 
 /* Reads host-side counters only (no device call, so a poll never waits behind a chunk in

@@ -763,21 +763,68 @@ __global__ __launch_bounds__(END_BLOCK) void k_chunk_end(DCtl* ctl_, const DChun
     }
 }
 
-/* src/renderer.cu:426-441 */
-__global__ __launch_bounds__(256) void k_tonemap(const float4* accum, ilm_pixel* out, int n, int spp, int op) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float4 a = gp(accum)[i];
+/* src/renderer.cu:426-441; the channels are whole numbers of 0..255 */
+__device__ inline void tonemap_px(const float4 a, int spp, int op, int& r, int& g, int& b) {
     float samples = (float)spp;
     V3 avg = mul3(mk3(a.x, a.y, a.z), 1 / samples);
     avg = tonemap_eval(op, avg);
     avg = mk3(__builtin_fmaxf(__builtin_fminf(avg.x, 1.0f), 0.0f), __builtin_fmaxf(__builtin_fminf(avg.y, 1.0f), 0.0f),
               __builtin_fmaxf(__builtin_fminf(avg.z, 1.0f), 0.0f));
+    r = (int)(255 * avg.x);
+    g = (int)(255 * avg.y);
+    b = (int)(255 * avg.z);
+}
+/* As ilm_pixel, 24 B per pixel. */
+__global__ __launch_bounds__(256) void k_tonemap(const float4* accum, ilm_pixel* out, int n, int spp, int op) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    int r, g, b;
+    tonemap_px(gp(accum)[i], spp, op, r, g, b);
     ilm_pixel px;
-    px.r = (uint64_t)(int)(255 * avg.x);
-    px.g = (uint64_t)(int)(255 * avg.y);
-    px.b = (uint64_t)(int)(255 * avg.z);
+    px.r = (uint64_t)r;
+    px.g = (uint64_t)g;
+    px.b = (uint64_t)b;
     gpw(out)[i] = px;
+}
+/* As one word per pixel, r | g << 8 | b << 16: what crosses PCIe, a sixth of the ilm_pixels that
+ * the host writes from it. With host not null the first thread also leaves the render's counters
+ * there (pinned host memory: segment total, then the two test counts). */
+__global__ __launch_bounds__(256) void k_tonemap8(const float4* accum, uint32_t* out, int n, int spp, int op,
+                                                  const unsigned long long* seg_total, const unsigned long long* trav,
+                                                  unsigned long long* host) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0 && host) {
+        gpw(host)[0] = gp(seg_total)[0];
+        gpw(host)[1] = gp(trav)[0];
+        gpw(host)[2] = gp(trav)[1];
+    }
+    if (i >= n) return;
+    int r, g, b;
+    tonemap_px(gp(accum)[i], spp, op, r, g, b);
+    gpw(out)[i] = (uint32_t)r | (uint32_t)g << 8 | (uint32_t)b << 16;
+}
+
+/* Results to pinned host memory, 16 B per pixel: the sums as packed RGB floats and the pixel words
+ * (either may be null). Bound by PCIe: 0.62 ms for 1920x1080 (54 GB/s, what a DMA of the same
+ * bytes takes), written directly so that no copy has to be queued behind the kernel. A thread
+ * takes four pixels, so that it writes whole 16-byte words; the outputs have room for n rounded
+ * up to four. */
+__global__ __launch_bounds__(256) void k_send(const float4* sums, const uint32_t* px, float* rgb_out, uint32_t* px_out, int n) {
+    const int i = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= n) return;
+    const int i1 = i + 1 < n ? i + 1 : i, i2 = i + 2 < n ? i + 2 : i, i3 = i + 3 < n ? i + 3 : i;
+    if (rgb_out) {
+        const GLOBAL float4* s = gp(sums);
+        const float4 a = s[i], b = s[i1], c = s[i2], d = s[i3];
+        GLOBAL float4* o = (GLOBAL float4*)(gpw(rgb_out) + 3 * (size_t)i);
+        o[0] = make_float4(a.x, a.y, a.z, b.x);
+        o[1] = make_float4(b.y, b.z, c.x, c.y);
+        o[2] = make_float4(c.z, d.x, d.y, d.z);
+    }
+    if (px_out) {
+        const GLOBAL uint32_t* p = gp(px);
+        *(GLOBAL uint4*)(gpw(px_out) + i) = make_uint4(p[i], p[i1], p[i2], p[i3]);
+    }
 }
 
 /* Kahan sums (float4 per pixel) to packed RGB floats, the layout of ilm_render's accum_rgb. */
@@ -792,6 +839,18 @@ __global__ __launch_bounds__(256) void k_sums_to_rgb(const float4* sums, float* 
 }
 
 __global__ void k_fill_zero4(float4* p, size_t n) {
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+        gpw(p)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+/* A render's first launch: its Kahan buffer cleared, the test counters too, and the segment total
+ * it starts from left in host[3] (pinned host memory). */
+__global__ void k_begin(float4* p, size_t n, const unsigned long long* seg_total, unsigned long long* trav, unsigned long long* host) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        gpw(host)[3] = gp(seg_total)[0];
+        gpw(trav)[0] = 0ull;
+        gpw(trav)[1] = 0ull;
+    }
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         gpw(p)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
@@ -904,6 +963,25 @@ hipError_t ilm_k_chunk_end(const KParams& P, unsigned long long* seg_total, int 
 hipError_t ilm_k_tonemap(const float4* accum, ilm_pixel* out, int n, int spp, int op, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     ILM_LAUNCH(k_tonemap, dim3((n + 255) / 256), dim3(256), 0, s, accum, out, n, spp, op);
+    return hipGetLastError();
+}
+hipError_t ilm_k_tonemap8(const float4* accum, uint32_t* out, int n, int spp, int op, const unsigned long long* seg_total,
+                          const unsigned long long* trav, unsigned long long* host, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    ILM_LAUNCH(k_tonemap8, dim3((n + 255) / 256), dim3(256), 0, s, accum, out, n, spp, op, seg_total, trav, host);
+    return hipGetLastError();
+}
+hipError_t ilm_k_send(const float4* sums, const uint32_t* px, float* rgb_out, uint32_t* px_out, int n, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    ILM_LAUNCH(k_send, dim3((n + 1023) / 1024), dim3(256), 0, s, sums, px, rgb_out, px_out, n);
+    return hipGetLastError();
+}
+hipError_t ilm_k_begin(float4* p, size_t n, const unsigned long long* seg_total, unsigned long long* trav,
+                       unsigned long long* host, hipStream_t s) {
+    size_t g = (n + 255) / 256;
+    if (g > 65535) g = 65535;
+    if (g < 1) g = 1;
+    ILM_LAUNCH(k_begin, dim3((unsigned)g), dim3(256), 0, s, p, n, seg_total, trav, host);
     return hipGetLastError();
 }
 hipError_t ilm_k_sums_to_rgb(const float4* sums, float* rgb, int n, hipStream_t s) {
