@@ -235,13 +235,13 @@ struct DChunk {
 /* Largest grid (one wave per workgroup) of k_finish. */
 #define ILM_TAIL_WAVES 8192
 
-/* Per-chunk control block (device). Cleared by k_ctl_init, never by a memset. */
+/* Per-chunk control block (device). Cleared by k_stage, never by a memset. */
 struct DCtl {
     uint32_t count[ILM_MAX_DEPTH + 2];   /* live paths entering depth d */
     uint32_t fetch[ILM_MAX_DEPTH + 2];   /* extend work cursor at depth d */
     unsigned long long segments;
     uint32_t total;
-    uint32_t pad;
+    uint32_t tail_n;                     /* waves of k_finish that had work */
     uint32_t tail[ILM_TAIL_WAVES];       /* segments each wave of k_finish traced */
 };
 

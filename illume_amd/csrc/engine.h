@@ -181,6 +181,7 @@ struct ilm_ctx {
 
     /* chunk descriptor staging */
     DChunk* h_chunk[ILM_RING] = {};
+    DChunk build{};                  /* the chunk being filled by run_jobs_sync (dev_mu) */
     hipEvent_t ring_ev[ILM_RING] = {};
     int ring_pos = 0;
     unsigned long long* h_u64 = nullptr;

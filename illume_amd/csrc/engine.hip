@@ -839,17 +839,24 @@ static bool packet_pays(const ilm_scene* s, const ilm_render_params& p, uint32_t
     return sgroup >= 2 && (double)s->inst_tris * 64.0 <= ILM_PACKET_MAX_TRIS * (double)sgroup * p.width * p.height;
 }
 
-/* Stage a chunk descriptor: pinned ring slot -> the device DChunk dst (ordered on stream s). */
-static int stage_chunk(ilm_ctx* ctx, const DChunk& hc, DChunk* dst, hipStream_t s) {
-    int slot = ctx->ring_pos++ % ILM_RING;
-    HIPTRY(ctx, hipEventSynchronize(ctx->ring_ev[slot]));
-    std::memcpy(ctx->h_chunk[slot], &hc, sizeof(DChunk));
-    HIPTRY(ctx, hipMemcpyAsync(dst, ctx->h_chunk[slot], sizeof(DChunk), hipMemcpyHostToDevice, s));
-    HIPTRY(ctx, hipEventRecord(ctx->ring_ev[slot], s));
+/* Stage a chunk descriptor: pinned ring slot -> pipeline q's device copy, on its stream, with the
+ * pipeline's queue counters (k_stage reads the slot itself). */
+static int stage_slot(ilm_ctx* ctx, int slot, int n_req, const Pipe& q) {
+    HIPTRY(ctx, ilm_k_stage(q.ctl, q.chunk, ctx->h_chunk[slot], n_req, ctx->h_chunk[slot]->n_work, q.stream));
+    HIPTRY(ctx, hipEventRecord(ctx->ring_ev[slot], q.stream));
     return ILM_OK;
 }
+static int stage_chunk(ilm_ctx* ctx, const DChunk& hc, int n_req, const Pipe& q) {
+    int slot = ctx->ring_pos++ % ILM_RING;
+    HIPTRY(ctx, hipEventSynchronize(ctx->ring_ev[slot]));
+    DChunk* d = ctx->h_chunk[slot];
+    std::memcpy(d, &hc, offsetof(DChunk, reqs));
+    std::memcpy(d->reqs, hc.reqs, (size_t)n_req * sizeof(DReq));
+    std::memcpy(d->work, hc.work, (size_t)hc.n_work * sizeof(DWork));
+    return stage_slot(ctx, slot, n_req, q);
+}
 
-/* A chunk's first launch after k_ctl_init. With per-step refill the first depth's extend and
+/* A chunk's first launch after k_stage. With per-step refill the first depth's extend and
  * shade form the camera rays where they use them, so only the per-path results are cleared
  * (by the packet extend itself when the first depth runs as packets); the other extend modes
  * read the rays k_raygen writes out. */
@@ -861,12 +868,11 @@ static hipError_t start_paths(ilm_ctx* ctx, const Pipe& q, KParams& P, hipStream
 }
 
 /* The launch sequence of one chunk with depth_steps depth iterations, in two parts: the depths
- * (ctl init, first rays, extend and shade per depth), then the accumulation into the requests'
+ * (first rays, extend and shade per depth, k_finish), then the accumulation into the requests'
  * Kahan sums and the segment count. */
 static int enqueue_depths(ilm_ctx* ctx, const Pipe& q, const KParams& base, int depth_steps, ProfileSink* prof) {
     hipStream_t s = q.stream;
     KParams P = base;
-    HIPTRY(ctx, ilm_k_ctl_init(P, s));
     HIPTRY(ctx, start_paths(ctx, q, P, s));
     for (int d = 0; d < (base.tail_only ? 0 : depth_steps); d++) {
         P.in = (d & 1) ? q.B : q.A;
@@ -891,15 +897,18 @@ static int enqueue_depths(ilm_ctx* ctx, const Pipe& q, const KParams& base, int 
     }
     return ILM_OK;
 }
-static int enqueue_finish(ilm_ctx* ctx, const Pipe& q, const KParams& base) {
-    HIPTRY(ctx, ilm_k_accumulate(base, ctx->gen_grid, q.stream));
-    HIPTRY(ctx, ilm_k_chunk_end(base, q.seg_total, base.quad_max > 0 ? ctx->fin_grid : 0, q.stream));
+/* blocks: enough for the chunk's pixels, 64 each (a captured graph serves chunks of any size) */
+static int acc_grid(const ilm_ctx* ctx, int64_t total_px) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>((total_px + 63) / 64, ctx->gen_grid * 4));
+}
+static int enqueue_finish(ilm_ctx* ctx, const Pipe& q, const KParams& base, int64_t total_px) {
+    HIPTRY(ctx, ilm_k_accumulate(base, acc_grid(ctx, total_px), q.seg_total, q.stream));
     return ILM_OK;
 }
 /* both parts, on one stream (debug paths and the allocation-free render) */
-static int enqueue_pipeline(ilm_ctx* ctx, const Pipe& q, const KParams& base, int depth_steps, ProfileSink* prof) {
+static int enqueue_pipeline(ilm_ctx* ctx, const Pipe& q, const KParams& base, int depth_steps, int64_t total_px, ProfileSink* prof) {
     int rc = enqueue_depths(ctx, q, base, depth_steps, prof);
-    return rc ? rc : enqueue_finish(ctx, q, base);
+    return rc ? rc : enqueue_finish(ctx, q, base, total_px);
 }
 
 /* whether every request of the chunk renders the same scene (the extend kernel then reads it
@@ -919,7 +928,7 @@ static int run_graph(ilm_ctx* ctx, int key, const Pipe& q, const KParams& P, int
         {
             std::lock_guard<std::mutex> cap(capture_mu(ctx->device));
             HIPTRY(ctx, hipStreamBeginCapture(q.stream, hipStreamCaptureModeThreadLocal));
-            int rc2 = finish ? enqueue_finish(ctx, q, P) : enqueue_depths(ctx, q, P, D, nullptr);
+            int rc2 = finish ? enqueue_finish(ctx, q, P, (int64_t)1 << 40) : enqueue_depths(ctx, q, P, D, nullptr);
             hipError_t ec = hipStreamEndCapture(q.stream, &g);
             if (rc2) return rc2;
             if (ec != hipSuccess) return fail(ctx, ILM_E_DEVICE, std::string("graph capture: ") + hipGetErrorString(ec));
@@ -941,7 +950,7 @@ static int launch_chunk(ilm_ctx* ctx, const DChunk& hc, const std::vector<Job*>&
     const int k = two ? ctx->next_pipe : 0;
     if (two) ctx->next_pipe ^= 1;
     const Pipe q = ctx_pipe(ctx, k);
-    int rc = stage_chunk(ctx, hc, q.chunk, q.stream);
+    int rc = stage_chunk(ctx, hc, (int)jobs.size(), q);
     if (rc) return rc;
     KParams P = base_params(ctx, q);
     const bool ovf = jobs_need_ovf(ctx, jobs);
@@ -955,8 +964,10 @@ static int launch_chunk(ilm_ctx* ctx, const DChunk& hc, const std::vector<Job*>&
             P.packet0 = packet_pays(j->scene, j->p, hc.work[w].sgroup) ? 1 : 0;
         }
     const int D = hc.depth_steps;
-    const bool graphs = ctx->opts.use_graphs && !prof && !ctx->opts.count_tests;
-    if (graphs) rc = run_graph(ctx, 2 * (64 * D + 32 * P.packet0 + 16 * (P.quad_max > 0) + 8 * P.tail_only + 4 * k + (uni ? 2 : 0) + (ovf ? 1 : 0)), q, P, D, false);
+    /* a chunk that k_finish does alone is two launches: launched directly, without the 15 us or so
+     * that starting two graphs takes */
+    const bool graphs = ctx->opts.use_graphs && !prof && !ctx->opts.count_tests && !P.tail_only;
+    if (graphs) rc = run_graph(ctx, 2 * (32 * D + 16 * P.packet0 + 8 * (P.quad_max > 0) + 4 * k + (uni ? 2 : 0) + (ovf ? 1 : 0)), q, P, D, false);
     else rc = enqueue_depths(ctx, q, P, D, prof);
     if (rc) return rc;
     if (ctx->npipes == 2) {
@@ -964,7 +975,7 @@ static int launch_chunk(ilm_ctx* ctx, const DChunk& hc, const std::vector<Job*>&
         if (k == 1) HIPTRY(ctx, hipStreamWaitEvent(q.stream, ctx->fill_ev, 0));
     }
     if (graphs) rc = run_graph(ctx, 2 * (2 * (P.quad_max > 0) + k) + 1, q, P, D, true);
-    else rc = enqueue_finish(ctx, q, P);
+    else rc = enqueue_finish(ctx, q, P, hc.total_px);
     if (rc) return rc;
     HIPTRY(ctx, hipEventRecord(ctx->acc_ev[k], q.stream));
     ctx->last_pipe = k;
@@ -1405,8 +1416,7 @@ static int run_jobs_sync(ilm_ctx* ctx, std::vector<Job*>& jobs, float* const* ac
     const hipEvent_t e0 = ctx->rend_ev[0], e1 = ctx->rend_ev[1];
     HIPTRY(ctx, hipEventRecord(e0, ctx->stream));
     if (ctx->stream2) HIPTRY(ctx, hipStreamWaitEvent(ctx->stream2, e0, 0));
-    DChunk* hc = new DChunk();
-    std::unique_ptr<DChunk> hc_own(hc);
+    DChunk* hc = &ctx->build;
     std::vector<Job*> in_chunk;
     int chunks = 0;
     int64_t max_paths = 0;
@@ -1628,15 +1638,14 @@ int ilm_render_noalloc(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* 
         if (!job_has_work(&j)) break;
         add_slice(ctx, &j, L.cap, 0, hc);
         hc.work[0].pass0 += params->first_sample;
-        HIPTRY(ctx, hipMemcpyAsync(q.chunk, &hc, sizeof(DChunk), hipMemcpyHostToDevice, ctx->stream));
-        HIPTRY(ctx, hipEventRecord(ctx->ring_ev[slot], ctx->stream));
+        if ((rc = stage_slot(ctx, slot, 1, q))) return rc;
         KParams P = base_params(ctx, q);
         P.trav_stats = nullptr;
         P.use_ovf = spill ? 1 : 0;
         P.uni_scene = 1;
         chunk_choices(ctx, hc.total_paths, scene_fits_quad(scene), P);
         if (ctx->opts.camera_packets == 0) P.packet0 = packet_pays(scene, *params, hc.work[0].sgroup) ? 1 : 0;
-        rc = enqueue_pipeline(ctx, q, P, hc.depth_steps, nullptr);
+        rc = enqueue_pipeline(ctx, q, P, hc.depth_steps, hc.total_px, nullptr);
         if (rc) return rc;
         chunks++;
         max_paths = std::max<int64_t>(max_paths, hc.total_paths);
@@ -1692,14 +1701,13 @@ int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int
         }
         hc->total_paths = (uint32_t)m;
         hc->depth_steps = 1;
-        int rc = stage_chunk(ctx, *hc, ctx->d_chunk, ctx->stream);
+        int rc = stage_chunk(ctx, *hc, 1, ctx_pipe(ctx));
         if (rc) return rc;
         HIPTRY(ctx, hipMemcpyAsync(ctx->A.o, o4.data(), m * sizeof(float4), hipMemcpyHostToDevice, ctx->stream));
         HIPTRY(ctx, hipMemcpyAsync(ctx->A.d, d4.data(), m * sizeof(float4), hipMemcpyHostToDevice, ctx->stream));
         KParams P = base_params(ctx);
         P.trav_stats = nullptr;
         P.use_ovf = scene_needs_ovf(ctx, scene) ? 1 : 0;
-        HIPTRY(ctx, ilm_k_ctl_init(P, ctx->stream));
         KParams F = P;
         chunk_choices(ctx, (uint32_t)m, scene_fits_quad(scene), F);
         if (F.tail_only) HIPTRY(ctx, ilm_k_extend_quad(P, 0, ctx->fin_grid, ctx->stream));
@@ -1749,7 +1757,7 @@ int ilm_debug_path_radiance(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_par
         int64_t m = std::min<int64_t>(ctx->cap, n - base);
         hc->total_paths = (uint32_t)m;
         hc->depth_steps = params->max_depth;
-        rc = stage_chunk(ctx, *hc, ctx->d_chunk, ctx->stream);
+        rc = stage_chunk(ctx, *hc, 1, ctx_pipe(ctx));
         if (rc) break;
         if (hipMemcpyAsync(d_list, pixel_pass + 2 * base, 2 * m * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream) != hipSuccess) {
             rc = fail(ctx, ILM_E_DEVICE, "list upload");

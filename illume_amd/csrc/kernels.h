@@ -2,15 +2,14 @@
 #pragma once
 #include "common.h"
 
-hipError_t ilm_k_ctl_init(const KParams& P, hipStream_t s);
+hipError_t ilm_k_stage(DCtl* ctl, DChunk* chunk, const DChunk* host, int n_req, int n_work, hipStream_t s);
 hipError_t ilm_k_raygen(const KParams& P, int grid, hipStream_t s);
 hipError_t ilm_k_extend(const KParams& P, int depth, int* ovf, int grid, hipStream_t s);
 hipError_t ilm_k_path_clear(const KParams& P, int grid, hipStream_t s);
 hipError_t ilm_k_shade(const KParams& P, int depth, int grid, hipStream_t s);
-hipError_t ilm_k_accumulate(const KParams& P, int grid, hipStream_t s);
+hipError_t ilm_k_accumulate(const KParams& P, int grid, unsigned long long* seg_total, hipStream_t s);
 hipError_t ilm_k_extend_quad(const KParams& P, int depth, int grid, hipStream_t s);
 hipError_t ilm_k_finish(const KParams& P, int grid, hipStream_t s);
-hipError_t ilm_k_chunk_end(const KParams& P, unsigned long long* seg_total, int tail_waves, hipStream_t s);
 hipError_t ilm_k_tonemap(const float4* accum, ilm_pixel* out, int n, int spp, int op, hipStream_t s);
 hipError_t ilm_k_tonemap8(const float4* accum, uint32_t* out, int n, int spp, int op, const unsigned long long* seg_total,
                           const unsigned long long* trav, unsigned long long* host, hipStream_t s);

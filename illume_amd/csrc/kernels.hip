@@ -1,7 +1,7 @@
 /*
  * kernels.hip - the gfx950 wavefront pipeline of the path tracer.
  *
- *   k_ctl_init     clear the chunk's queue counters (no memset: graph-safe)
+ *   k_stage        fetch the chunk's descriptor and clear its queue counters (no copy, no memset)
  *   k_raygen       camera rays for (request, pass, pixel) work, PCG32 seeded per path
  *                  (src/renderer.cu:61-69,81-110)
  *   k_extend       closest hit (traverse.h): spheres, then a TLAS over instances and per-mesh
@@ -11,8 +11,8 @@
  *                  is the compaction: wave ballot + one atomic per wave appends survivors to
  *                  the next depth's queue (replaces the host round trip of
  *                  src/renderer.cu:390-424)
- *   k_accumulate   Kahan-compensated per-pixel sum of the chunk's path radiances, in pass order
- *   k_chunk_end    segment count (src/renderer.cu:554)
+ *   k_accumulate   Kahan-compensated per-pixel sum of the chunk's path radiances, in pass order,
+ *                  and the chunk's segment count (src/renderer.cu:554)
  *   k_tonemap      src/renderer.cu:426-441 with src/tonemapper.cu:42-76
  *
  * Every kernel reads its work count from device memory, so a whole chunk is a fixed launch
@@ -38,20 +38,33 @@
  * 75. 4 and 6 waves measured within 1 % of 5 on queues that fit, 6 slower on the smallest. */
 #define FIN_WPE 5
 
-__global__ void k_ctl_init(DCtl* ctl_, const DChunk* chunk) {
+/* The chunk's descriptor, read from pinned host memory (the parts in use: a few hundred bytes of
+ * its 58 KB for a plain render, so one trip over PCIe), and its queue counters. One block; a queued
+ * copy of the whole and a launch of its own for the counters took 15 us more per chunk. */
+#define STAGE_BLOCK 256
+__global__ __launch_bounds__(STAGE_BLOCK) void k_stage(DCtl* ctl_, DChunk* chunk_, const DChunk* host_, int n_req, int n_work) {
     GLOBAL DCtl* ctl = gpw(ctl_);
-    for (int i = threadIdx.x; i < ILM_MAX_DEPTH + 2; i += blockDim.x) {
-        ctl->count[i] = 0u;
+    GLOBAL uint32_t* dst = (GLOBAL uint32_t*)gpw(chunk_);
+    const GLOBAL uint32_t* src = (const GLOBAL uint32_t*)gp(host_);
+    const uint32_t head = (uint32_t)(offsetof(DChunk, reqs) / 4) + (uint32_t)n_req * (uint32_t)(sizeof(DReq) / 4);
+    const uint32_t all = head + (uint32_t)n_work * (uint32_t)(sizeof(DWork) / 4);
+    const uint32_t total = gp(host_)->total_paths;
+    for (uint32_t i = threadIdx.x; i < all; i += STAGE_BLOCK) {
+        const uint32_t w = i < head ? i : (uint32_t)(offsetof(DChunk, work) / 4) + i - head;
+        dst[w] = src[w];
+    }
+    for (int i = threadIdx.x; i < ILM_MAX_DEPTH + 2; i += STAGE_BLOCK) {
+        ctl->count[i] = i == 0 ? total : 0u;
         ctl->fetch[i] = 0u;
     }
-    __syncthreads();
     if (threadIdx.x == 0) {
-        const uint32_t total = gp(chunk)->total_paths;
-        ctl->count[0] = total;
         ctl->total = total;
         ctl->segments = 0ull;
+        ctl->tail_n = 0u;
     }
 }
+static_assert(sizeof(DReq) % 4 == 0 && sizeof(DWork) % 4 == 0 && offsetof(DChunk, reqs) % 4 == 0 && offsetof(DChunk, work) % 4 == 0,
+              "copied by words");
 
 /* src/renderer.cu:81-110 (and the per-pass seeding of :61-69): the camera rays written out, for
  * the extend modes that read the first depth's rays from memory */
@@ -648,7 +661,38 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FIN_WPE, 8))
             __syncthreads();
         }
     }
-    if (lane == 0) ctl->tail[blockIdx.x] = segs;
+    if (lane == 0 && blockIdx.x * per < count) ctl->tail[blockIdx.x] = segs;
+    if (lane == 0 && blockIdx.x == 0) {
+        const uint32_t waves = (count + per - 1u) / per;
+        ctl->tail_n = waves < gridDim.x ? waves : gridDim.x;
+    }
+}
+
+/* Segments of the chunk (one wave): the queues the per-depth kernels traced (with k_finish, those
+ * longer than quad_max), and what k_finish's waves traced, eight loads in flight per lane. */
+__device__ inline void chunk_end(GLOBAL DCtl* ctl, int D, unsigned long long* seg_total, int quad_max) {
+    const uint32_t lane = threadIdx.x;
+    unsigned long long s = 0;
+    for (int d = (int)lane; d < D; d += 64) {
+        const uint32_t c = ctl->count[d];
+        if (c > (uint32_t)quad_max) s += c;
+    }
+    const uint32_t n = quad_max > 0 ? ctl->tail_n : 0u;
+    for (uint32_t w0 = 0; w0 < n; w0 += 512u) {
+        uint32_t v[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++) {
+            const uint32_t w = w0 + k * 64u + lane;
+            v[k] = w < n ? ctl->tail[w] : 0u;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++) s += v[k];
+    }
+    for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d);
+    if (lane == 0) {
+        ctl->segments = s;
+        atomicAdd(gpw(seg_total), s);   /* chunks of the two pipelines may end together */
+    }
 }
 
 /* Kahan-compensated sum of the chunk's path radiances, pass order per pixel. One wave per
@@ -657,7 +701,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FIN_WPE, 8))
  * least 8 long, the wave reads each 8-pass batch of its pixels cooperatively: 8 lanes per pixel
  * read that pixel's 128 contiguous bytes, so a load instruction touches 8 cache lines rather than
  * 64, and the batch is handed to the pixel's lane through LDS. Otherwise each lane reads its own
- * pixel's radiances. Either way a lane adds its pixel's passes in pass order. */
+ * pixel's radiances. Either way a lane adds its pixel's passes in pass order. The grid's last block
+ * counts the chunk's segments instead: a launch of its own for that added 6 us to every chunk. */
 #define ACC_BATCH 8
 #define ACC_ROW (ACC_BATCH + 1)   /* float4 per pixel row in LDS: one pad against bank conflicts */
 __device__ inline void kahan_add(float4& s, float4& c, const float4 x) {
@@ -666,14 +711,19 @@ __device__ inline void kahan_add(float4& s, float4& c, const float4 x) {
     y = x.y - c.y; t = s.y + y; c.y = (t - s.y) - y; s.y = t;
     y = x.z - c.z; t = s.z + y; c.z = (t - s.z) - y; s.z = t;
 }
-__global__ __launch_bounds__(64) void k_accumulate(KParams P) {
+__global__ __launch_bounds__(64) void k_accumulate(KParams P, unsigned long long* seg_total) {
     __shared__ float4 stage[64 * ACC_ROW];
     const GLOBAL DChunk* C = gp(P.chunk);
+    const uint32_t blocks = gridDim.x - 1u;
+    if (blockIdx.x == blocks) {
+        chunk_end(gpw(P.ctl), C->depth_steps, seg_total, P.quad_max);
+        return;
+    }
     const uint32_t total_px = C->total_px;
     const GLOBAL float4* contrib = gp(P.contrib);
     const uint32_t lane = threadIdx.x;
     /* the loop bound is uniform over the wave: every lane reaches the LDS barriers */
-    for (uint32_t g0 = blockIdx.x * 64u; g0 < total_px; g0 += gridDim.x * 64u) {
+    for (uint32_t g0 = blockIdx.x * 64u; g0 < total_px; g0 += blocks * 64u) {
         const uint32_t g = g0 + lane;
         const bool valid = g < total_px;
         const uint32_t gq = valid ? g : g0;
@@ -735,31 +785,6 @@ __global__ __launch_bounds__(64) void k_accumulate(KParams P) {
             acc[p] = s;
             cmp[p] = c;
         }
-    }
-}
-
-/* Segments of the chunk: the queues the per-depth kernels traced (all of them, or with k_finish
- * (tail_waves > 0) those longer than quad_max), and what k_finish's waves traced. */
-#define END_BLOCK 512
-__global__ __launch_bounds__(END_BLOCK) void k_chunk_end(DCtl* ctl_, const DChunk* chunk, unsigned long long* seg_total,
-                                                         int quad_max, int tail_waves) {
-    __shared__ unsigned long long part[END_BLOCK / 64];
-    GLOBAL DCtl* ctl = gpw(ctl_);
-    const int t = threadIdx.x;
-    const int D = gp(chunk)->depth_steps;
-    unsigned long long s = 0;
-    for (int d = t; d < D; d += END_BLOCK) {
-        const uint32_t c = ctl->count[d];
-        if (tail_waves == 0 || c > (uint32_t)quad_max) s += c;
-    }
-    for (int w = t; w < tail_waves; w += END_BLOCK) s += ctl->tail[w];
-    for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d);
-    if ((t & 63) == 0) part[t >> 6] = s;
-    __syncthreads();
-    if (t == 0) {
-        for (int w = 1; w < END_BLOCK / 64; w++) s += part[w];
-        ctl->segments = s;
-        atomicAdd(gpw(seg_total), s);   /* chunks of the two pipelines may end together */
     }
 }
 
@@ -866,8 +891,8 @@ __global__ void k_begin(float4* p, size_t n, const unsigned long long* seg_total
         hipLaunchKernelGGL(__VA_ARGS__);                                                           \
     } while (0)
 
-hipError_t ilm_k_ctl_init(const KParams& P, hipStream_t s) {
-    ILM_LAUNCH(k_ctl_init, dim3(1), dim3(256), 0, s, P.ctl, P.chunk);
+hipError_t ilm_k_stage(DCtl* ctl, DChunk* chunk, const DChunk* host, int n_req, int n_work, hipStream_t s) {
+    ILM_LAUNCH(k_stage, dim3(1), dim3(STAGE_BLOCK), 0, s, ctl, chunk, host, n_req, n_work);
     return hipGetLastError();
 }
 hipError_t ilm_k_raygen(const KParams& P, int grid, hipStream_t s) {
@@ -937,8 +962,8 @@ hipError_t ilm_k_shade(const KParams& P, int depth, int grid, hipStream_t s) {
     else ILM_LAUNCH((k_shade<0, 0>), dim3(grid), dim3(SHADE_BLOCK), 0, s, P, depth);
     return hipGetLastError();
 }
-hipError_t ilm_k_accumulate(const KParams& P, int grid, hipStream_t s) {
-    ILM_LAUNCH(k_accumulate, dim3(grid * 4), dim3(64), 0, s, P);
+hipError_t ilm_k_accumulate(const KParams& P, int grid, unsigned long long* seg_total, hipStream_t s) {
+    ILM_LAUNCH(k_accumulate, dim3(grid + 1), dim3(64), 0, s, P, seg_total);
     return hipGetLastError();
 }
 hipError_t ilm_k_extend_quad(const KParams& P, int depth, int grid, hipStream_t s) {
@@ -954,10 +979,6 @@ hipError_t ilm_k_finish(const KParams& P, int grid, hipStream_t s) {
         if (P.uni_scene) ILM_LAUNCH((k_finish<0, 1>), dim3(grid), dim3(64), 0, s, P);
         else ILM_LAUNCH((k_finish<0, 0>), dim3(grid), dim3(64), 0, s, P);
     }
-    return hipGetLastError();
-}
-hipError_t ilm_k_chunk_end(const KParams& P, unsigned long long* seg_total, int tail_waves, hipStream_t s) {
-    ILM_LAUNCH(k_chunk_end, dim3(1), dim3(END_BLOCK), 0, s, P.ctl, P.chunk, seg_total, P.quad_max, tail_waves);
     return hipGetLastError();
 }
 hipError_t ilm_k_tonemap(const float4* accum, ilm_pixel* out, int n, int spp, int op, hipStream_t s) {

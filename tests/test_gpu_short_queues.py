@@ -103,3 +103,20 @@ def test_camera_rays_per_lane_and_as_packets_match(w, h, spp, layout):
     for a, px, info in out[1:]:
         assert np.array_equal(a, out[0][0], equal_nan=True) and np.array_equal(px, out[0][1])
         assert info["segments"] == out[0][2]["segments"]
+
+
+@pytest.mark.parametrize("graphs", [0, 1])
+def test_descriptors_of_any_length_are_staged(graphs):
+    """Chunks of 1, 33 and 64 requests after one another: only the parts in use of a chunk's
+    descriptor reach the device, and what an earlier chunk left there is not read."""
+    spec, st = S.tiny_mesh_scene()
+    ps = [render_params(**dict(st, width=3 + 5 * (i % 9), height=2 + i, spp=1 + i % 4, max_depth=2 + i % 5)) for i in range(64)]
+    with illume_amd.Context(0, use_graphs=graphs) as c:
+        s = c.scene(spec)
+        alone = [c.render(s, p) for p in ps]
+        for n in (64, 1, 33, 64, 1):
+            res, info = c.render_batch([s] * n, ps[:n])
+            for (a, px), ref in zip(res, alone):
+                assert np.array_equal(a, ref[0], equal_nan=True) and np.array_equal(px, ref[1])
+            assert info["segments"] == sum(r[2]["segments"] for r in alone[:n])
+        s.free()
