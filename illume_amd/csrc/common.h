@@ -235,10 +235,14 @@ struct DChunk {
 /* Largest grid (one wave per workgroup) of k_finish. */
 #define ILM_TAIL_WAVES 8192
 
+/* Bands of the first depth's path ids that k_extend_packet hands out by cursors of their own. */
+#define ILM_BANDS 8
+
 /* Per-chunk control block (device). Cleared by k_stage, never by a memset. */
 struct DCtl {
     uint32_t count[ILM_MAX_DEPTH + 2];   /* live paths entering depth d */
     uint32_t fetch[ILM_MAX_DEPTH + 2];   /* extend work cursor at depth d */
+    uint32_t band[ILM_BANDS][32];        /* the packet kernel's cursors, [b][0], a cache line each */
     unsigned long long segments;
     uint32_t total;
     uint32_t tail_n;                     /* waves of k_finish that had work */

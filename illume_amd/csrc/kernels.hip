@@ -57,6 +57,7 @@ __global__ __launch_bounds__(STAGE_BLOCK) void k_stage(DCtl* ctl_, DChunk* chunk
         ctl->count[i] = i == 0 ? total : 0u;
         ctl->fetch[i] = 0u;
     }
+    if (threadIdx.x < ILM_BANDS) ctl->band[threadIdx.x][0] = 0u;
     if (threadIdx.x == 0) {
         ctl->total = total;
         ctl->segments = 0ull;

@@ -763,11 +763,59 @@ __device__ inline uint32_t pool_fetch(uint32_t count, uint32_t fetch) {
     return share < fetch ? share : fetch;
 }
 
-/* First depth with per-step refill: each wave reserves consecutive path ids (P.ext_fetch per
- * queue atomic, less for a queue that is short for the grid or drains), and traces them 64 at a
- * time: forms their camera rays (camera_ray) and walks one packet per distinct scene among them.
+/* First depth with per-step refill: each wave reserves consecutive path ids and traces them 64 at
+ * a time: forms their camera rays (camera_ray) and walks one packet per distinct scene among them.
  * Every path id of the chunk passes through here once, so the kernel also clears the per-path
- * results (the chunk needs no separate clear). */
+ * results (the chunk needs no separate clear).
+ *
+ * Reservations are P.ext_fetch ids, less when the queue is short for the grid or drains. Atomics on
+ * one cache line serialise, 11.4 ns each over the whole device, and a packet is cheap: one cursor's
+ * 262144 reservations held the 67 M camera rays of the 1024x1024x64 metal scene at 3.2 ms. So the
+ * ids are cut in ILM_BANDS bands with a cursor line each (1.8 ns per atomic over eight lines: 2.6
+ * ms); a wave begins in the band of its workgroup's XCD and, when that is used up, goes on in the
+ * next one that has ids left. */
+struct Bands {
+    uint32_t count, size, fetch;   /* ids, ids per band (whole batches), the largest reservation */
+};
+__device__ inline uint32_t band_waves(uint32_t b) { return (gridDim.x + (uint32_t)(ILM_BANDS - 1) - b) / ILM_BANDS; }
+__device__ inline uint32_t band_len(const Bands& B, uint32_t b) {
+    const uint32_t s = b * B.size;
+    return s >= B.count ? 0u : B.count - s < B.size ? B.count - s : B.size;
+}
+/* the wave's next ids [pos, end), or false when no band has ids left; band and want are its state */
+__device__ inline bool band_next(GLOBAL DCtl* ctl, const Bands& B, uint32_t& band, uint32_t& want, bool first_trip,
+                                 uint32_t& pos, uint32_t& end) {
+    const int lane = threadIdx.x;
+    for (;; first_trip = false) {
+        const uint32_t n = band_len(B, band), waves = band_waves(band), first = waves * B.fetch;
+        /* a wave's first reservation is fixed by its index; the cursor hands out the rest */
+        uint32_t at = (blockIdx.x / ILM_BANDS) * B.fetch;
+        if (!first_trip) {
+            at = n;
+            if (first < n) {
+                uint32_t k = 0;
+                if (lane == 0) k = atomicAdd(&ctl->band[band][0], want);
+                at = first + (uint32_t)uni_i((int)k);
+            }
+        }
+        if (at < n) {
+            const uint32_t e = n - at < want ? n : at + want;
+            pos = band * B.size + at;
+            end = band * B.size + e;
+            const uint32_t g = ((n - e) / (2u * waves)) & ~(uint32_t)(EXT_BLOCK - 1);
+            want = g < (uint32_t)EXT_BLOCK ? (uint32_t)EXT_BLOCK : (g > B.fetch ? B.fetch : g);
+            return true;
+        }
+        /* lane b looks at band b; a cursor only grows, so a band found used up stays so */
+        const uint32_t b = (uint32_t)lane % ILM_BANDS;
+        const uint32_t k = __hip_atomic_load((uint32_t*)&ctl->band[b][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t left = (uint32_t)__ballot(band_waves(b) * B.fetch + k < band_len(B, b)) & ((1u << ILM_BANDS) - 1u);
+        if (!left) return false;
+        band = (band + (uint32_t)__builtin_ctz(left >> band | left << (ILM_BANDS - band))) % ILM_BANDS;
+        want = (uint32_t)EXT_BLOCK;
+    }
+}
+
 template <int TRI, int QUANT, int COUNT>
 __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_extend_packet(KParams P, int depth) {
     __shared__ int stk[PKT_STACK];
@@ -775,40 +823,20 @@ __global__ __launch_bounds__(EXT_BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8)
     GLOBAL DCtl* ctl = gpw(P.ctl);
     const uint32_t count = ctl->count[depth];
     if (count <= (uint32_t)P.quad_max) return;   /* left to k_finish */
-    const uint32_t fetch = pool_fetch(count, (uint32_t)P.ext_fetch);
+    const Bands bands = {count, ((count + ILM_BANDS * EXT_BLOCK - 1u) / (ILM_BANDS * EXT_BLOCK)) * EXT_BLOCK,
+                         pool_fetch(count, (uint32_t)P.ext_fetch)};
     const GLOBAL DReq* reqs = gp(P.chunk)->reqs;
     TravCount tc = {0u, 0u};
-    const uint32_t guide = gridDim.x * 2u;
     CamSrc cs;
     const bool cu = camsrc_load(P, cs);
     const uint64_t su = cu ? cs.s : 0ull;
-    /* the first reservation is fixed by the wave's index; the cursor hands out the rest (one
-     * address's atomics serialise, so a wave with nothing to do should not touch it) */
-    const uint32_t first = gridDim.x * fetch;
-    uint32_t want = fetch;
-    uint32_t b = 0, end = 0;
+    uint32_t band = blockIdx.x % ILM_BANDS, want = bands.fetch, pos = 0, end = 0;
     bool first_trip = true;
-    for (;;) {
-        if (b >= end) {
-            uint32_t base = 0;
-            if (first_trip) {
-                base = blockIdx.x * fetch;
-                first_trip = false;
-            } else {
-                if (first >= count) break;
-                if (lane == 0) base = atomicAdd(&ctl->fetch[depth], want);
-                base = first + (uint32_t)uni_i((int)__shfl(base, 0));
-            }
-            if (base >= count) break;
-            b = base;
-            end = base + want < count ? base + want : count;
-            const uint32_t left = count - end;
-            const uint32_t g = (left / guide) & ~(uint32_t)(EXT_BLOCK - 1);
-            want = g < (uint32_t)EXT_BLOCK ? (uint32_t)EXT_BLOCK : (g > fetch ? fetch : g);
-        }
-        const uint32_t r = b + (uint32_t)lane;
+    for (;; first_trip = false) {
+        if (pos >= end && !band_next(ctl, bands, band, want, first_trip, pos, end)) break;
+        const uint32_t r = pos + (uint32_t)lane;
         const bool valid = r < end;
-        b += (uint32_t)EXT_BLOCK;
+        pos += (uint32_t)EXT_BLOCK;
         if (valid) {
             gpw(P.contrib)[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (P.seg_count) gpw(P.seg_count)[r] = 0;

@@ -88,7 +88,8 @@ def test_closest_hits_of_short_queues_match(pair, n):
 
 
 @pytest.mark.parametrize("layout", ["fp32", "quant8"])
-@pytest.mark.parametrize("w,h,spp", [(1024, 512, 1), (1024, 512, 2), (333, 331, 8), (96, 64, 64), (700, 701, 3)])
+@pytest.mark.parametrize("w,h,spp", [(1024, 512, 1), (1024, 512, 2), (333, 331, 8), (96, 64, 64), (700, 701, 3),
+                                     (1001, 703, 6)])
 def test_camera_rays_per_lane_and_as_packets_match(w, h, spp, layout):
     """The default choice between packets and lanes for the first depth, and both by name, over
     queues of few and many rays per wave (whole and split, ragged, one to 64 samples a pixel)."""
