@@ -264,6 +264,10 @@ LayoutF make_layout_f(const std::vector<BNode>& nodes, int root) {
                 f.c[k].a = ch[k].a;
                 f.c[k].b = make_float4(ch[k].lz, ch[k].hz, 0.0f, 0.0f);
             }
+            if (code == ILM_NO_CHILD) {   /* a box no ray enters when the planes are taken by its direction */
+                f.c[k].a = make_float4(ILM_FLT_MAX, -ILM_FLT_MAX, ILM_FLT_MAX, -ILM_FLT_MAX);
+                f.c[k].b = make_float4(ILM_FLT_MAX, -ILM_FLT_MAX, 0.0f, 0.0f);
+            }
             std::memcpy(&f.c[k].b.z, &code, 4);
         }
         L.nodes.push_back(f);

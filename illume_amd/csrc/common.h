@@ -50,7 +50,7 @@ struct __attribute__((aligned(128))) FNode {
     struct Child {
         float4 a;           /* lo.x hi.x lo.y hi.y */
         float4 b;           /* lo.z hi.z child code bits, 0 */
-    } c[4];                 /* unused slots: code ILM_NO_CHILD */
+    } c[4];                 /* unused slots: code ILM_NO_CHILD, box FLT_MAX..-FLT_MAX */
 };
 static_assert(sizeof(FNode) == 128, "FNode is one 128-byte line");
 /* stack entries per quad of that walk; scenes with a larger bound are not given to it */
@@ -284,6 +284,7 @@ struct KParams {
     int shade_sort;         /* shade each block's paths in shading-key order (staged in LDS) */
     int cam0;               /* the first depth forms camera rays in extend and shade (no raygen) */
     int packet0;            /* ... and its extend traces each wave's camera rays as one packet */
+    int packet_f;           /* the packets walk FNodes: one scene, whose walk fits ILM_QUAD_STACK */
     int uni_scene;          /* every request of the chunk renders the same scene */
     int tail_only;          /* the whole chunk fits quad_max: no per-depth launches */
     int quad_max;           /* queues of at most this many rays go to the quad walk (0: none) */

@@ -822,21 +822,26 @@ static KParams base_params(ilm_ctx* ctx) { return base_params(ctx, ctx_pipe(ctx)
 static void chunk_choices(const ilm_ctx* ctx, uint32_t total_paths, bool quad_fits, KParams& P) {
     const bool quad = quad_fits && ctx->opts.extend_mode == ILM_EXTEND_DEFAULT && !ctx->opts.profile && !ctx->opts.count_tests;
     P.quad_max = quad ? ILM_TAIL_PATHS : 0;
+    P.packet_f = quad_fits && P.uni_scene ? 1 : 0;
     P.tail_only = (int64_t)total_paths <= (int64_t)P.quad_max ? 1 : 0;
 }
 
 /* Whether a request's camera rays are traced as packets by default. A packet visits the union of
  * its 64 rays' walks, and one wave carries it to its end, so it pays while the 64 / sgroup pixels
  * it covers show few triangles; the scene's triangles per image pixel stand for that. First-depth
- * time as packets / per lane, 8-bit nodes (FP32 nodes within 0.1, except where given), by
- * triangles in the footprint: 100k triangles at 1920x1080 0.90 (0.8, 4 samples), 1.01 (1.6, 2),
- * 1.10 (3.2, 1); at 640x480 1.03 (2.6, 8), 1.06 (5, 4), 1.29 (10, 2; FP32 1.12), 1.57 (21, 1);
- * 11 small meshes 0.81 (2.4, 4), 0.97 (4.8, 2), 1.23 (9.6, 1); 525k triangles 0.97 (3, 16), 1.04
- * (6, 8), 1.07 (12, 4), 1.66 (24, 2); 12 instances of 722k 0.99 (19, 32; FP32 0.87), 1.27 (37,
- * 16), 1.77 (150, 4), 4.2 (600, 1). */
+ * time as packets over FNodes / per lane with 8-bit nodes, by triangles in the footprint: 100k
+ * triangles at 1920x1080 0.74 (0.4, 8 samples), 0.76 (1.6, 2), 0.88 (3.1, 1); at 640x480 0.67 (2.6,
+ * 8), 0.72 (5, 4), 0.90 (10, 2), 1.09 (21, 1); 11 small meshes 0.70 (4.4, 8), 0.83 (8.8, 4), 0.94
+ * (18, 2), 1.23 (35, 1); 32k triangles at 320x240 0.82 (6.7, 4), 0.94 (13, 2), 0.95 (27, 1); 12
+ * instances of 722k 0.69 (9.4, 64), 0.80 (19, 32), 1.04 (38, 16), 1.32 (75, 8), 4.0 (600, 1). At one
+ * sample the 64 pixels differ more (32k triangles at 400x300, three passes: 1.11 at 17), so the line
+ * lies at half the triangles there; packets over the other layouts (several scenes in a chunk, very
+ * deep trees) cost about a fifth more and lose at one sample. */
 #define ILM_PACKET_MAX_TRIS 20
-static bool packet_pays(const ilm_scene* s, const ilm_render_params& p, uint32_t sgroup) {
-    return sgroup >= 2 && (double)s->inst_tris * 64.0 <= ILM_PACKET_MAX_TRIS * (double)sgroup * p.width * p.height;
+static bool packet_pays(const ilm_scene* s, const ilm_render_params& p, uint32_t sgroup, bool fnodes) {
+    if (sgroup < 2 && !fnodes) return false;
+    const double limit = sgroup < 2 ? 0.5 * ILM_PACKET_MAX_TRIS : ILM_PACKET_MAX_TRIS;
+    return (double)s->inst_tris * 64.0 <= limit * (double)sgroup * p.width * p.height;
 }
 
 /* Stage a chunk descriptor: pinned ring slot -> pipeline q's device copy, on its stream, with the
@@ -961,13 +966,13 @@ static int launch_chunk(ilm_ctx* ctx, const DChunk& hc, const std::vector<Job*>&
     if (ctx->opts.camera_packets == 0)
         for (int w = 0; w < hc.n_work && P.packet0; w++) {
             const Job* j = jobs[hc.work[w].req];
-            P.packet0 = packet_pays(j->scene, j->p, hc.work[w].sgroup) ? 1 : 0;
+            P.packet0 = packet_pays(j->scene, j->p, hc.work[w].sgroup, P.packet_f) ? 1 : 0;
         }
     const int D = hc.depth_steps;
     /* a chunk that k_finish does alone is two launches: launched directly, without the 15 us or so
      * that starting two graphs takes */
     const bool graphs = ctx->opts.use_graphs && !prof && !ctx->opts.count_tests && !P.tail_only;
-    if (graphs) rc = run_graph(ctx, 2 * (32 * D + 16 * P.packet0 + 8 * (P.quad_max > 0) + 4 * k + (uni ? 2 : 0) + (ovf ? 1 : 0)), q, P, D, false);
+    if (graphs) rc = run_graph(ctx, 2 * (64 * D + 32 * P.packet_f + 16 * P.packet0 + 8 * (P.quad_max > 0) + 4 * k + (uni ? 2 : 0) + (ovf ? 1 : 0)), q, P, D, false);
     else rc = enqueue_depths(ctx, q, P, D, prof);
     if (rc) return rc;
     if (ctx->npipes == 2) {
@@ -1644,7 +1649,7 @@ int ilm_render_noalloc(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* 
         P.use_ovf = spill ? 1 : 0;
         P.uni_scene = 1;
         chunk_choices(ctx, hc.total_paths, scene_fits_quad(scene), P);
-        if (ctx->opts.camera_packets == 0) P.packet0 = packet_pays(scene, *params, hc.work[0].sgroup) ? 1 : 0;
+        if (ctx->opts.camera_packets == 0) P.packet0 = packet_pays(scene, *params, hc.work[0].sgroup, P.packet_f) ? 1 : 0;
         rc = enqueue_pipeline(ctx, q, P, hc.depth_steps, hc.total_px, nullptr);
         if (rc) return rc;
         chunks++;

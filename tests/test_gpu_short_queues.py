@@ -121,3 +121,27 @@ def test_descriptors_of_any_length_are_staged(graphs):
                 assert np.array_equal(a, ref[0], equal_nan=True) and np.array_equal(px, ref[1])
             assert info["segments"] == sum(r[2]["segments"] for r in alone[:n])
         s.free()
+
+
+@pytest.mark.parametrize("name", ["cornell", "tiny", "gold", "medium"])
+@pytest.mark.parametrize("tri", ["mt", "watertight"])
+@pytest.mark.parametrize("w,h,spp", [(65, 63, 1), (61, 67, 7), (40, 30, 64)])
+def test_packets_over_fnodes_match_lanes(name, tri, w, h, spp):
+    """Packets whose directions share an octant and packets that straddle an axis (the image's middle,
+    rotated and unrotated instances), last packets that are not full, spheres; one scene and several."""
+    spec, st = SCENES[name]()
+    other, _ = S.tiny_mesh_scene(n=3)
+    p = render_params(**dict(st, width=w, height=h, spp=spp, max_depth=2))
+    out = []
+    for packets in (1, 2):
+        with illume_amd.Context(0, extend_mode=3, camera_packets=packets, tri_test=tri) as c:
+            s, t = c.scene(spec), c.scene(other)
+            both, info = c.render_batch([s, t, s], [p, p, p])
+            out.append((c.render(s, p), both, info["segments"]))
+            s.free()
+            t.free()
+    (a, b) = out
+    assert np.array_equal(a[0][0], b[0][0], equal_nan=True) and np.array_equal(a[0][1], b[0][1])
+    assert a[0][2]["segments"] == b[0][2]["segments"] and a[2] == b[2]
+    for x, y in zip(a[1], b[1]):
+        assert np.array_equal(x[0], y[0], equal_nan=True) and np.array_equal(x[1], y[1])
