@@ -145,3 +145,29 @@ def test_packets_over_fnodes_match_lanes(name, tri, w, h, spp):
     assert a[0][2]["segments"] == b[0][2]["segments"] and a[2] == b[2]
     for x, y in zip(a[1], b[1]):
         assert np.array_equal(x[0], y[0], equal_nan=True) and np.array_equal(x[1], y[1])
+
+
+@pytest.mark.parametrize("scenes,opts", [(2, {}), (6, {}), (2, dict(sched_fair=1)), (2, dict(pipes=1)), (2, dict(chunk_passes=3))])
+def test_requests_of_several_scenes_in_chunks_of_their_own(scenes, opts):
+    """Work of 2^19 paths and more per scene runs as one chunk per scene while few scenes have work, and
+    joined otherwise: the images and the segment count are those of the requests alone either way."""
+    names = ["tiny", "cornell", "gold", "tiny", "cornell", "tiny"][:scenes]
+    with illume_amd.Context(0, **opts) as c:
+        sc = [c.scene(SCENES[n]()[0]) for n in names]
+        ps = [render_params(**dict(SCENES[n]()[1], width=400 + 8 * i, height=300, spp=6 - i % 3, max_depth=4 + i))
+              for i, n in enumerate(names)]
+        sc, ps = sc + sc[:1], ps + [render_params(**dict(SCENES["tiny"]()[1], width=31, height=17, spp=3, max_depth=5))]
+        alone = [c.render(s, p) for s, p in zip(sc, ps)]
+        res, info = c.render_batch(sc, ps)
+        hs = [c.submit(s, p) for s, p in zip(sc, ps)]
+        served = []
+        for h in hs:
+            h.wait(60000)
+            served.append(h.result())
+            h.free()
+        for (a, px), (b, bx), ref in zip(res, served, alone):
+            for x, y in ((a, ref[0]), (b, ref[0]), (px, ref[1]), (bx, ref[1])):
+                assert np.array_equal(x, y, equal_nan=x.dtype == np.float32)
+        assert info["segments"] == sum(r[2]["segments"] for r in alone)
+        for s in sc[:-1]:
+            s.free()
