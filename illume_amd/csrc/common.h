@@ -286,6 +286,8 @@ struct KParams {
     int packet0;            /* ... and its extend traces each wave's camera rays as one packet */
     int packet_f;           /* the packets walk FNodes: one scene, whose walk fits ILM_QUAD_STACK */
     int uni_scene;          /* every request of the chunk renders the same scene */
+    unsigned long long* report;   /* pinned host words, one per depth, or null: k_shade leaves the */
+    uint32_t report_tag;          /* count of its queue there (tag << 32 | count) */
     int tail_only;          /* the whole chunk fits quad_max: no per-depth launches */
     int quad_max;           /* queues of at most this many rays go to the quad walk (0: none) */
 };

@@ -184,6 +184,8 @@ struct ilm_ctx {
     DChunk build{};                  /* the chunk being filled by run_jobs_sync (dev_mu) */
     hipEvent_t ring_ev[ILM_RING] = {};
     int ring_pos = 0;
+    unsigned long long* h_report = nullptr;   /* pinned: counts the depths of a chunk report, by tag */
+    uint32_t report_tag = 0;
     unsigned long long* h_u64 = nullptr;
 
     std::map<int, hipGraphExec_t> graphs;

@@ -445,6 +445,9 @@ __global__ SHADE_BOUNDS void k_shade(KParams P, int depth) {
     __shared__ uint32_t s_out[SHADE_WAVES * OUT_KEYS];
     GLOBAL DCtl* ctl = gpw(P.ctl);
     const uint32_t count = ctl->count[depth];
+    if (P.report && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(P.report + depth, (unsigned long long)P.report_tag << 32 | count, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     if (count <= (uint32_t)P.quad_max) return;   /* left to k_finish (every thread of the grid leaves) */
     const GLOBAL DReq* reqs = gp(P.chunk)->reqs;
     /* a chunk of one scene: its arrays are read once per block */

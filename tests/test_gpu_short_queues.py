@@ -171,3 +171,41 @@ def test_requests_of_several_scenes_in_chunks_of_their_own(scenes, opts):
         assert info["segments"] == sum(r[2]["segments"] for r in alone)
         for s in sc[:-1]:
             s.free()
+
+
+def test_renders_that_follow_their_counts_match_when_interleaved():
+    """Renders whose depths are launched by the counts of the depths before them: one after another with
+    other depths and sizes (a count left by an earlier render is not taken for a later one's), from two
+    threads on two contexts, against contexts that launch every depth."""
+    import threading
+    reqs = [("medium", 400, 300, 3, 45), ("tiny", 520, 510, 1, 2), ("medium", 512, 513, 1, 3), ("tiny", 400, 300, 3, 4),
+            ("cornell", 512, 513, 1, 5), ("medium", 333, 251, 7, 45), ("tiny", 640, 480, 2, 12)]
+    with illume_amd.Context(0, extend_mode=3) as c:
+        sc = {k: c.scene(SCENES[k]()[0]) for k in SCENES}
+        ref = [c.render(sc[r[0]], render_params(**dict(SCENES[r[0]]()[1], width=r[1], height=r[2], spp=r[3], max_depth=r[4])))
+               for r in reqs]
+        for s in sc.values():
+            s.free()
+    bad = []
+
+    def work(order):
+        with illume_amd.Context(0) as c:
+            sc = {k: c.scene(SCENES[k]()[0]) for k in SCENES}
+            for i in order:
+                k, w, h, spp, depth = reqs[i]
+                p = render_params(**dict(SCENES[k]()[1], width=w, height=h, spp=spp, max_depth=depth))
+                for call in (c.render, c.render_noalloc):
+                    a, px, info = call(sc[k], p)
+                    if not (np.array_equal(a, ref[i][0], equal_nan=True) and np.array_equal(px, ref[i][1]) and
+                            info["segments"] == ref[i][2]["segments"]):
+                        bad.append((call.__name__, reqs[i]))
+            for s in sc.values():
+                s.free()
+
+    n = len(reqs)
+    ts = [threading.Thread(target=work, args=(o,)) for o in (list(range(n)) * 2, list(range(n))[::-1] * 2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
