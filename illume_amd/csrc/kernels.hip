@@ -8,15 +8,17 @@
  *                  BLAS, stack walk in wave64 with the stack in LDS, t-pruned and ordered
  *                  (src/renderer.cu:112-137, src/primitives/mesh.cu:479-562)
  *   k_shade        medium free flight and the 9 BSDFs (src/renderer.cu:139-388); its epilogue
- *                  is the compaction: wave ballot + one atomic per wave appends survivors to
+ *                  is the compaction: ballots + one atomic per block append survivors to
  *                  the next depth's queue (replaces the host round trip of
  *                  src/renderer.cu:390-424)
+ *   k_finish       the rest of a chunk once a queue is short, four lanes per ray (quad.h)
  *   k_accumulate   Kahan-compensated per-pixel sum of the chunk's path radiances, in pass order,
  *                  and the chunk's segment count (src/renderer.cu:554)
  *   k_tonemap      src/renderer.cu:426-441 with src/tonemapper.cu:42-76
+ *   k_begin, k_send  a request's sums cleared; its results into pinned memory
  *
  * Every kernel reads its work count from device memory, so a whole chunk is a fixed launch
- * sequence (capturable as a hipGraph) with no host synchronisation between depths.
+ * sequence (capturable as a hipGraph) that waits for nothing on the host between depths.
  */
 #include "quad.h"
 

@@ -760,7 +760,7 @@ __device__ inline void packet_trace(const GLOBAL DScene* S, V3 O, V3 D, Best& B,
  * sign, which is the rule, the near and far planes are known and a child takes 18 vector instructions
  * (24 otherwise). The BLAS walk is a loop of its own: one loop over both spaces kept two sets of ray
  * registers and copied them 30 instructions a trip. First depth of the 1024x1024x64 metal scene 2.60
- * -> 2.21 ms, of 12 instances of 722k triangles at 1280x720x64 7.5 -> 6.0 ms. */
+ * -> 2.21 ms, of 12 instances of 722k triangles at 1280x720x64 7.1 -> 5.7 ms. */
 typedef int I16v __attribute__((ext_vector_type(16)));
 typedef int I4v __attribute__((ext_vector_type(4)));
 __device__ inline V3 i3(int a, int b, int c) { return mk3(__int_as_float(a), __int_as_float(b), __int_as_float(c)); }
