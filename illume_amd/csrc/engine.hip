@@ -40,8 +40,13 @@ static thread_local std::string g_err;
  * descriptor, traversal-stack spill area, Kahan sums and pixels of one render, all carved from
  * this array. Each GPU the library runs on holds its own copy until the process ends. In host
  * code the name is a host-side stand-in, never a device address: kernels and copies use the
- * address hipGetSymbolAddress gives for the current device (noalloc_scratch_of). */
-static __device__ __align__(256) unsigned char scratch[ILM_NOALLOC_SCRATCH_BYTES];
+ * address hipGetSymbolAddress gives for the current device (noalloc_scratch_of). The control
+ * block's packet cursors and k_finish counts lie beyond ILM_NOALLOC_SCRATCH_BYTES, so that the
+ * largest image the array takes does not depend on how many waves those kernels run. */
+#define ILM_NOALLOC_CTL_BYTES (sizeof(DCtl::band) + sizeof(DCtl::tail))
+#define ILM_NOALLOC_ARRAY_BYTES (ILM_NOALLOC_SCRATCH_BYTES + ILM_NOALLOC_CTL_BYTES)
+static_assert(ILM_NOALLOC_CTL_BYTES % 256 == 0, "the blocks behind the control block keep their places in the documented bytes");
+static __device__ __align__(256) unsigned char scratch[ILM_NOALLOC_ARRAY_BYTES];
 
 #define ILM_MAX_DEVICES 64
 static std::mutex g_scratch_mu;                     /* g_scratch_ptr */
@@ -1645,9 +1650,9 @@ static bool noalloc_layout(const ilm_ctx* ctx, int64_t wh, bool spill, NoallocLa
     L.off_accum = o;  o = align256(o + 2 * (size_t)wh * sizeof(float4));
     L.off_px = o;     o = align256(o + (size_t)wh * sizeof(ilm_pixel));
     L.off_paths = o;
-    if (o >= (size_t)ILM_NOALLOC_SCRATCH_BYTES) return false;
+    if (o >= ILM_NOALLOC_ARRAY_BYTES) return false;
     /* 9 arrays, each rounded up to 256 B */
-    const size_t room = (size_t)ILM_NOALLOC_SCRATCH_BYTES - o;
+    const size_t room = ILM_NOALLOC_ARRAY_BYTES - o;
     if (room < 9 * 256) return false;
     int64_t cap = (int64_t)((room - 9 * 256) / ILM_PATH_BYTES);
     cap = std::min<int64_t>(cap & ~(int64_t)63, cap_of(ctx->opts));
@@ -1694,7 +1699,7 @@ int ilm_render_noalloc(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* 
         q.hits.h = (float4*)take(n * sizeof(float4));
         q.hits.inst = (int*)take(n * sizeof(int));
         q.contrib = (float4*)take(n * sizeof(float4));
-        if (pp > base + (size_t)ILM_NOALLOC_SCRATCH_BYTES) return fail(ctx, ILM_E_DEVICE, "scratch carving overflow");
+        if (pp > base + ILM_NOALLOC_ARRAY_BYTES) return fail(ctx, ILM_E_DEVICE, "scratch carving overflow");
     }
     /* the array keeps the previous call's contents: the Kahan buffer and the segment counter
      * start at zero; the control block is cleared by every chunk's first kernel */

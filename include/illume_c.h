@@ -341,9 +341,10 @@ int ilm_render(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params,
  * outputs as ilm_render (bit-identical accum_rgb and pixels, same segment count), but every
  * device buffer of the call - path state, hits, per-path results, control block, chunk
  * descriptor, traversal-stack spill area, Kahan sums and pixels - is carved from one static
- * device array of ILM_NOALLOC_SCRATCH_BYTES per GPU, which each GPU the library runs on holds
- * until the process ends. The call makes no hipMalloc/hipFree and no host allocation, launches
- * kernels directly (no graph) and synchronises before it returns.
+ * device array of ILM_NOALLOC_SCRATCH_BYTES (and 33 KB of queue cursors and counts) per GPU,
+ * which each GPU the library runs on holds until the process ends. The call makes no
+ * hipMalloc/hipFree and no host allocation, launches kernels directly (no graph) and
+ * synchronises before it returns.
  * Limit: W*H*56 bytes of pixel buffers plus at least 4096 paths (148 bytes each), and for a
  * scene whose BVH needs the spilling traversal stack a spill area of up to 28 MB, must fit the
  * array (up to about 2.38 M pixels, 1.87 M with the spill area); larger images return
