@@ -76,6 +76,7 @@ struct StagePool {
     std::mutex mu;                          /* leaf lock */
     std::vector<Staging*> free;
     size_t bytes = 0, cap = (size_t)256 << 20;
+    std::atomic<int64_t> largest{INT64_MAX};    /* larger buffers are refused (ilm_debug_pinned_limit) */
 };
 
 struct Job {

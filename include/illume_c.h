@@ -331,7 +331,11 @@ const char* ilm_loader_error(void);
 
 /* ---- plain render (one request, synchronous) ----
  * accum_rgb: W*H*3 floats, Kahan-compensated sum of the spp sample radiances (nullable).
- * out: W*H pixels after tonemapping, as src/renderer.cu:426-441 (nullable). */
+ * out: W*H pixels after tonemapping, as src/renderer.cu:426-441 (nullable).
+ * Results travel through pinned host memory: 16 bytes a pixel, at most 64 MB at a time here and in
+ * ilm_render_batch, the whole image for a served request. The context keeps up to 256 MB of it for
+ * later calls until it is closed. Where the system has none, these two copy into pageable memory
+ * instead (same results, slower); ilm_submit returns ILM_E_NOMEM. */
 int ilm_render(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params,
                float* accum_rgb, ilm_pixel* out, ilm_render_info* info);
 
@@ -402,6 +406,9 @@ int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int
  * segments: n (nullable) - number of closest-hit queries each path made. */
 int ilm_debug_path_radiance(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params,
                             const uint32_t* pixel_pass, int32_t n, float* rgb, int32_t* segments);
+/* From now on no pinned buffer of more than `bytes` can be had for this context's results, as on a
+ * system that refuses it (buffers kept idle are freed; 0: none at all). */
+int ilm_debug_pinned_limit(ilm_ctx* ctx, int64_t bytes);
 /* Instance i's matrices as the device uses them: out[0..15] object-to-world, [16..31] inverse,
  * [32..47] inverse-transpose (row-major). */
 int ilm_debug_instance_matrices(const ilm_scene* scene, int32_t i, float* out48);
