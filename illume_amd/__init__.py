@@ -66,6 +66,7 @@ def lib():
         "ilm_bvh_export": (C.c_int, [vp, P(C.c_float), P(C.c_int32), P(C.c_int32), P(C.c_int32), P(C.c_int32)]),
         "ilm_bvh_quantized_size": (C.c_int, [vp, P(C.c_int32), P(C.c_int32), P(C.c_int32)]),
         "ilm_bvh_export_quantized": (C.c_int, [vp, P(C.c_float), P(C.c_float), P(C.c_int32)]),
+        "ilm_bvh_export_fnodes": (C.c_int, [vp, P(C.c_int32), P(C.c_int32), P(C.c_int32), P(C.c_float), P(C.c_int32)]),
         "ilm_bvh_free": (None, [vp]),
         "ilm_debug_closest_hit": (C.c_int, [vp, vp, P(C.c_float), C.c_int32, P(C.c_int32), P(C.c_int32), P(C.c_float)]),
         "ilm_debug_path_radiance": (C.c_int, [vp, vp, P(RenderParams), P(C.c_uint32), C.c_int32, P(C.c_float), P(C.c_int32)]),
@@ -357,9 +358,14 @@ def bvh_build(positions, indices):
         ex = np.empty((max(nq.value, 1), 4, 6), np.float32)
         ch = np.empty((max(nq.value, 1), 4), np.int32)
         L.ilm_bvh_export_quantized(h, _fp(qb), _fp(ex), _ip(ch))
+        nf, froot, levels = C.c_int32(), C.c_int32(), C.c_int32()
+        L.ilm_bvh_export_fnodes(h, C.byref(nf), C.byref(froot), C.byref(levels), None, None)
+        fb = np.empty((nf.value, 4, 6), np.float32)
+        fc = np.empty((nf.value, 4), np.int32)
+        L.ilm_bvh_export_fnodes(h, None, None, None, _fp(fb), _ip(fc))
         return dict(info=struct_to_dict(info), boxes=boxes, children=children, leaf_first=first, leaf_count=count,
                     order=order, q_boxes=qb[:nq.value], q_exact=ex[:nq.value], q_child=ch[:nq.value],
-                    q_root=root.value, q_depth=qd.value)
+                    q_root=root.value, q_depth=qd.value, f_boxes=fb, f_child=fc, f_root=froot.value, f_levels=levels.value)
     finally:
         L.ilm_bvh_free(h)
 

@@ -83,6 +83,27 @@ extern "C" int ilm_bvh_export_quantized(const ilm_bvh* b, float* qboxes, float* 
     return ILM_OK;
 }
 
+/* The FNode layout of the same tree: per FNode 4 children's boxes (lo.xyz, hi.xyz) and codes. */
+extern "C" int ilm_bvh_export_fnodes(const ilm_bvh* b, int32_t* num_fnodes, int32_t* root, int32_t* levels, float* boxes,
+                                     int32_t* child) {
+    if (!b) return ILM_E_INVALID;
+    const Layout2 l2 = make_layout2(b->tree);
+    const LayoutF f = make_layout_f(l2.nodes, l2.root);
+    if (num_fnodes) *num_fnodes = (int32_t)f.nodes.size();
+    if (root) *root = f.root;
+    if (levels) *levels = f.levels;
+    for (size_t i = 0; i < f.nodes.size(); i++)
+        for (int k = 0; k < 4; k++) {
+            const FNode::Child& c = f.nodes[i].c[k];
+            if (boxes) {
+                const float v[6] = {c.a.x, c.a.z, c.b.x, c.a.y, c.a.w, c.b.y};
+                std::memcpy(boxes + 24 * i + 6 * k, v, sizeof(v));
+            }
+            if (child) std::memcpy(child + 4 * i + k, &c.b.z, 4);
+        }
+    return ILM_OK;
+}
+
 extern "C" void ilm_bvh_free(ilm_bvh* b) { delete b; }
 
 /* The device layouts ilm_scene_upload would use for this mesh, built or loaded from cache_dir

@@ -387,6 +387,12 @@ int ilm_bvh_export(const ilm_bvh* b, float* boxes, int32_t* children, int32_t* l
  * the child code (child: >= 0 node, leaf code with bit 31 set, 0x7fffffff unused). */
 int ilm_bvh_quantized_size(const ilm_bvh* b, int32_t* num_qnodes, int32_t* root, int32_t* max_depth);
 int ilm_bvh_export_quantized(const ilm_bvh* b, float* qboxes, float* exact, int32_t* child);
+/* FP32 BVH4 layout (the walk with four lanes per ray, the camera packets) collapsed from the FP32
+ * BVH2 nodes: node count, root child code and nodes on the longest path from the root; per node and
+ * child k < 4 the box (24 floats per node; unused: FLT_MAX .. -FLT_MAX) and the child code as above.
+ * Null arrays only query. */
+int ilm_bvh_export_fnodes(const ilm_bvh* b, int32_t* num_fnodes, int32_t* root, int32_t* levels, float* boxes,
+                          int32_t* child);
 void ilm_bvh_free(ilm_bvh* b);
 /* Device layouts (FP32 BVH2 nodes, 8-bit BVH4 nodes, leaf triangle order) exactly as
  * ilm_scene_upload builds them, through the BVH cache in cache_dir (NULL: none). Replaces the
