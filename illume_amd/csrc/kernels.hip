@@ -390,6 +390,7 @@ __device__ inline uint32_t split_rank(uint32_t key, uint32_t* tab) {
     }
     const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
     if (lane < NK) tab[wid * NK + lane] = 0u;
+    wave_lds_order();   /* the count of a key replaces the zero that another lane wrote */
     if (rank == 0u) tab[wid * NK + (int)key] = (uint32_t)__popcll(m);
     return rank;
 }

@@ -43,6 +43,14 @@ __device__ inline int quad_add(int v) {
     return v + qperm_i<QP_XOR2>(v);
 }
 
+/* Between LDS accesses of different lanes of a wave: the LDS serves a wave's accesses in order, so
+ * nothing has to be waited for, but the compiler, which follows one lane, must not move or forward
+ * them across. No instruction. */
+__device__ inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 /* A wave's rays and their hits in LDS: up to 64 rays staged by the lanes that own them and taken
  * by the quads one at a time; a finished quad leaves the hit in the ray's own columns. */
 struct QuadLds {
@@ -93,6 +101,7 @@ __device__ inline void quad_walk(LDSAS QuadLds* L, int n, const GLOBAL DReq* req
     best_init(B);
     O = D = o = d = id = mk3(0.0f, 0.0f, 0.0f);
     for (;;) {
+        wave_lds_order();   /* a stack entry is read by the lanes of its quad, written by one of them in an earlier trip */
         const unsigned long long idle = __ballot(ridx < 0);
         if (next < n) {
             if (idle) {
