@@ -70,6 +70,7 @@ def lib():
         "ilm_bvh_free": (None, [vp]),
         "ilm_debug_closest_hit": (C.c_int, [vp, vp, P(C.c_float), C.c_int32, P(C.c_int32), P(C.c_int32), P(C.c_float)]),
         "ilm_debug_path_radiance": (C.c_int, [vp, vp, P(RenderParams), P(C.c_uint32), C.c_int32, P(C.c_float), P(C.c_int32)]),
+        "ilm_debug_depths_to_launch": (C.c_int, [P(C.c_uint32), C.c_int32, C.c_int32, C.c_int32, C.c_uint32]),
         "ilm_debug_pinned_limit": (C.c_int, [vp, C.c_int64]),
         "ilm_debug_instance_matrices": (C.c_int, [vp, C.c_int32, P(C.c_float)]),
     }

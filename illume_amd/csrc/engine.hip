@@ -911,41 +911,74 @@ static hipError_t start_paths(ilm_ctx* ctx, const Pipe& q, KParams& P, hipStream
     return P.cam0 ? ilm_k_path_clear(P, ctx->gen_grid, s) : ilm_k_raygen(P, ctx->gen_grid, s);
 }
 
-/* The count of the queue that k_shade found at `depth` (left in h_report with the chunk's tag). */
+/* The count of the queue that k_shade found at `depth`, if it is there (in h_report with the chunk's
+ * tag). */
+static bool report_there(const KParams& P, int depth, uint32_t& count) {
+    const unsigned long long v = __atomic_load_n(P.report + depth, __ATOMIC_RELAXED);
+    count = (uint32_t)v;
+    return (uint32_t)(v >> 32) == P.report_tag;
+}
+/* The same, waited for. The thread keeps its processor: what it waits for is at most one depth away
+ * from leaving the GPU idle, and on a busy host a yield gives away several milliseconds. */
 static int wait_report(ilm_ctx* ctx, const Pipe& q, const KParams& P, int depth, uint32_t& count) {
     for (unsigned spin = 1;; spin++) {
         const bool look = (spin & 255u) == 0;
         const hipError_t e = look ? hipStreamQuery(q.stream) : hipErrorNotReady;
-        const unsigned long long v = __atomic_load_n(P.report + depth, __ATOMIC_RELAXED);
-        if ((uint32_t)(v >> 32) == P.report_tag) {
-            count = (uint32_t)v;
-            return ILM_OK;
-        }
+        if (report_there(P, depth, count)) return ILM_OK;
         if (e == hipSuccess) return fail(ctx, ILM_E_DEVICE, "a depth ended without its count");
         if (e != hipErrorNotReady) HIPTRY(ctx, e);
         if (look) (void)hipGetLastError();
-        if ((spin & 63u) == 0) std::this_thread::yield();
     }
+}
+
+/* How many of a chunk's D depths to have launched in all, when `launched` are and the first `known`
+ * (two or more) have reported their counts. Once a queue is at most `limit`, no more. Otherwise at once
+ * all whose queues are still longer than `limit` if each is shorter than the one before by the ratio
+ * of the last two known, whose launches need no further word from the host, and the two after them
+ * that would be launched while their counts are waited for. A host that finds every launched depth reported came late, the GPU is about to
+ * run dry or has, and it will be late again: all of them, as if nothing were reported. */
+static int depths_to_launch(const uint32_t* count, int known, int launched, int D, uint32_t limit) {
+    const uint32_t last = count[known - 1];
+    if (last <= limit) return launched;
+    const double ratio = (double)last / (double)std::max(1u, count[known - 2]);
+    if (known >= launched || ratio >= 1.0) return D;
+    const double more = std::ceil(std::log((double)limit / last) / std::log(ratio)) - 1.0;
+    return (int)std::min<double>(D, known + more + 2.0);
+}
+int ilm_debug_depths_to_launch(const uint32_t* counts, int32_t known, int32_t launched, int32_t depth_steps, uint32_t limit) {
+    if (!counts || known < 2 || known > launched || launched > depth_steps || limit == 0) return ILM_E_INVALID;
+    return depths_to_launch(counts, known, launched, depth_steps, limit);
 }
 
 /* The launch sequence of one chunk with depth_steps depth iterations, in two parts: the depths
  * (first rays, extend and shade per depth, k_finish), then the accumulation into the requests'
  * Kahan sums and the segment count.
  *
- * With P.report the depths are launched two ahead of the counts that k_shade reports, and no more of
- * them once a queue is left to k_finish: the two launches of a depth with nothing to do take 9 us, and
- * a render of 45 depths whose queue is short after four spent 0.37 of its 2.5 ms on the others. */
+ * With P.report the depths are launched ahead of the counts that k_shade reports, and no more of them
+ * once a queue is left to k_finish (depths_to_launch): the two launches of a depth with nothing to do
+ * take 9 us, and a render of 45 depths whose queue is short after four spent 0.37 of its 2.5 ms on the
+ * others. On a host whose processor is shared with one and with three busy threads that render takes 4.0
+ * and 8.0 ms of wall time at the median (7.2 and 15.7 with all depths launched ahead through a graph,
+ * 16 and 32 with two depths ahead and a thread that yields), a 1024x1024, 16 spp, depth 16 one 10.8 and
+ * 19.3 (22 and 48, 20 and 40). */
 static int enqueue_depths(ilm_ctx* ctx, const Pipe& q, const KParams& base, int depth_steps, ProfileSink* prof) {
     const bool follow = base.report != nullptr;
     hipStream_t s = q.stream;
     KParams P = base;
     HIPTRY(ctx, start_paths(ctx, q, P, s));
-    for (int d = 0; d < (base.tail_only ? 0 : depth_steps); d++) {
-        if (follow && d >= 3) {
-            uint32_t count = 0;
-            int rc = wait_report(ctx, q, P, d - 2, count);
-            if (rc) return rc;
-            if (count <= (uint32_t)P.quad_max) break;
+    int goal = base.tail_only ? 0 : follow ? std::min(3, depth_steps) : depth_steps;
+    uint32_t counts[ILM_MAX_DEPTH];
+    int known = 0;
+    for (int d = 0;; d++) {
+        if (d == goal) {
+            if (!follow || goal == depth_steps) break;
+            for (; known < d - 1; known++) {
+                const int rc = wait_report(ctx, q, P, known, counts[known]);
+                if (rc) return rc;
+            }
+            if (report_there(P, known, counts[known])) known++;
+            goal = depths_to_launch(counts, known, d, depth_steps, (uint32_t)P.quad_max);
+            if (goal == d) break;
         }
         P.in = (d & 1) ? q.B : q.A;
         P.out = (d & 1) ? q.A : q.B;

@@ -412,6 +412,10 @@ int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int
  * segments: n (nullable) - number of closest-hit queries each path made. */
 int ilm_debug_path_radiance(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params,
                             const uint32_t* pixel_pass, int32_t n, float* rgb, int32_t* segments);
+/* How many of a chunk's depth_steps depths the library would have launched next (the rule is beside its
+ * code, no device is used): `launched` are, counts holds the paths that entered the first `known` of
+ * them, and a queue of at most `limit` paths needs no more. */
+int ilm_debug_depths_to_launch(const uint32_t* counts, int32_t known, int32_t launched, int32_t depth_steps, uint32_t limit);
 /* From now on no pinned buffer of more than `bytes` can be had for this context's results, as on a
  * system that refuses it (buffers kept idle are freed; 0: none at all). */
 int ilm_debug_pinned_limit(ilm_ctx* ctx, int64_t bytes);
