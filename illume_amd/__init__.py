@@ -69,6 +69,7 @@ def lib():
         "ilm_bvh_export_fnodes": (C.c_int, [vp, P(C.c_int32), P(C.c_int32), P(C.c_int32), P(C.c_float), P(C.c_int32)]),
         "ilm_bvh_free": (None, [vp]),
         "ilm_debug_closest_hit": (C.c_int, [vp, vp, P(C.c_float), C.c_int32, P(C.c_int32), P(C.c_int32), P(C.c_float)]),
+        "ilm_debug_closest_hit_quad": (C.c_int, [vp, vp, P(C.c_float), C.c_int32, P(C.c_int32), P(C.c_int32), P(C.c_float)]),
         "ilm_debug_path_radiance": (C.c_int, [vp, vp, P(RenderParams), P(C.c_uint32), C.c_int32, P(C.c_float), P(C.c_int32)]),
         "ilm_debug_depths_to_launch": (C.c_int, [P(C.c_uint32), C.c_int32, C.c_int32, C.c_int32, C.c_uint32]),
         "ilm_debug_pinned_limit": (C.c_int, [vp, C.c_int64]),
@@ -214,13 +215,16 @@ class Context:
         _check(lib().ilm_stats_get(self.h, C.byref(s)), self.h)
         return struct_to_dict(s)
 
-    def closest_hit(self, scene, rays):
+    def closest_hit(self, scene, rays, quad=False):
+        """Closest hits (instance, primitive, distance) of world-space rays by the context's extend kernel,
+        or with quad=True by the walk with four lanes per ray that finishes short queues."""
         rays = np.ascontiguousarray(rays, dtype=np.float32).reshape(-1, 6)
         n = rays.shape[0]
         inst = np.empty(n, np.int32)
         prim = np.empty(n, np.int32)
         t = np.empty(n, np.float32)
-        _check(lib().ilm_debug_closest_hit(self.h, scene.h, _fp(rays), n, _ip(inst), _ip(prim), _fp(t)), self.h)
+        hits = lib().ilm_debug_closest_hit_quad if quad else lib().ilm_debug_closest_hit
+        _check(hits(self.h, scene.h, _fp(rays), n, _ip(inst), _ip(prim), _fp(t)), self.h)
         return inst, prim, t
 
     def path_radiance(self, scene, params, pixel_pass):

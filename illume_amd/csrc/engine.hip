@@ -1867,10 +1867,12 @@ int ilm_render_noalloc(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* 
 
 /* ======================= parity hooks ======================= */
 
-int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int32_t n, int32_t* inst,
-                          int32_t* prim, float* t) {
+/* quad: by the walk of short queues (quad.h); otherwise by the extend kernel of the context's options */
+static int closest_hits(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int32_t n, int32_t* inst, int32_t* prim, float* t,
+                        bool quad) {
     if (!ctx || !scene || !rays || n < 0 || !inst || !prim || !t) return fail(ctx, ILM_E_INVALID, "bad arguments");
     if (int rc = check_scene_stack(ctx, scene)) return rc;
+    if (quad && !scene_fits_quad(scene)) return fail(ctx, ILM_E_UNSUPPORTED, "BVH too deep for the walk with four lanes per ray");
     std::lock_guard<std::mutex> dev(ctx->dev_mu);
     HIPTRY(ctx, hipSetDevice(ctx->device));
     std::unique_ptr<DChunk> hc(new DChunk());
@@ -1896,9 +1898,7 @@ int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int
         KParams P = base_params(ctx);
         P.trav_stats = nullptr;
         P.use_ovf = scene_needs_ovf(ctx, scene) ? 1 : 0;
-        KParams F = P;
-        chunk_choices(ctx, (uint32_t)m, scene_fits_quad(scene), F);
-        if (F.tail_only) HIPTRY(ctx, ilm_k_extend_quad(P, 0, ctx->fin_grid, ctx->stream));
+        if (quad) HIPTRY(ctx, ilm_k_extend_quad(P, 0, ctx->fin_grid, ctx->stream));
         else HIPTRY(ctx, ilm_k_extend(P, 0, ctx->ovf, ctx->ext_grid, ctx->stream));
         h4.resize(m);
         hi.resize(m);
@@ -1914,6 +1914,13 @@ int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int
         }
     }
     return ILM_OK;
+}
+
+int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int32_t n, int32_t* inst, int32_t* prim, float* t) {
+    return closest_hits(ctx, scene, rays, n, inst, prim, t, false);
+}
+int ilm_debug_closest_hit_quad(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int32_t n, int32_t* inst, int32_t* prim, float* t) {
+    return closest_hits(ctx, scene, rays, n, inst, prim, t, true);
 }
 
 int ilm_debug_pinned_limit(ilm_ctx* ctx, int64_t bytes) {

@@ -408,6 +408,11 @@ int ilm_bvh_device_layouts(const ilm_mesh_desc* m, const char* cache_dir, int32_
  * or -1 for a miss; prim: triangle index within the instance's mesh (-1 otherwise); t: hit distance. */
 int ilm_debug_closest_hit(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int32_t n,
                           int32_t* inst, int32_t* prim, float* t);
+/* The same hits by the walk that finishes short queues (four lanes per ray, FP32 BVH4 nodes whatever
+ * bvh_layout says) instead of the context's extend kernel; ILM_E_UNSUPPORTED for a scene too deep for
+ * its stacks, which no render gives it. */
+int ilm_debug_closest_hit_quad(ilm_ctx* ctx, ilm_scene* scene, const float* rays, int32_t n,
+                               int32_t* inst, int32_t* prim, float* t);
 /* Radiance of single paths (pixel, pass) with the render's RNG stream; rgb: n*3;
  * segments: n (nullable) - number of closest-hit queries each path made. */
 int ilm_debug_path_radiance(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params,
