@@ -267,7 +267,8 @@ def bench_plain(args):
         _, _, info = ctx.render(scene, p, want_accum=False)
         log("warmup %d: %.1f ms, %d segments" % (i, info["device_ms"], info["segments"]))
 
-    # timed steps: each render one replay of its captured graphs
+    # timed steps: a render of one chunk is launched directly, its depths ahead of the counts they
+    # report; one of several chunks replays captured graphs
     segs = 0
     lat = []
     dev_ms = 0.0

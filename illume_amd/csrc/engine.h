@@ -87,7 +87,7 @@ struct Job {
     uint32_t* d_px = nullptr;       /* pixel words (k_tonemap8) */
     size_t accum_cap = 0, px_cap = 0;   /* allocation sizes (pool buffers may be larger) */
     BufPool* pool = nullptr;
-    int64_t bytes = 0;              /* device bytes while admitted */
+    int64_t bytes = 0;              /* charged to the HBM budget while admitted */
     int next_pass = 0;              /* issue cursor: pass, pixel */
     int64_t next_px = 0;
     int64_t split_npx = 0;          /* > 0: issued as pixel ranges of this many slots, all passes each */

@@ -1,13 +1,13 @@
 /*
  * engine.hip - host runtime behind the C ABI: context, device-resident scenes, the chunked
- * wavefront driver (direct launches or one hipGraph per depth count), the plain, batched and
- * served forms, and the parity hooks.
+ * wavefront driver (direct launches, or hipGraphs by depth count and kind of chunk), the plain,
+ * batched and served forms, and the parity hooks.
  *
  * Reference counterparts: Renderer::render_to_bitmap (src/renderer.cu:498-597) and
  * SceneRef (src/scene/sceneref.cpp:9-148). Differences by design: scenes stay on the device
  * across renders, path state is struct-of-arrays and compacted on the device, many passes
- * (and many requests) share one chunk of launches, and nothing synchronises with the host
- * between depths.
+ * (and many requests) share one chunk of launches, and no depth synchronises with the host: its
+ * launches are queued ahead of it.
  */
 #include <algorithm>
 #include <atomic>
@@ -2197,6 +2197,8 @@ int ilm_submit(ilm_ctx* ctx, ilm_scene* scene, const ilm_render_params* params, 
     Job* j = new Job();
     j->scene = scene;
     j->p = *params;
+    /* what admission charges: sums, compensations and a whole ilm_pixel, 56 B a pixel, although the
+     * device holds the pixel as a 4-byte word; what fits a budget and what is refused stays as it was */
     j->bytes = wh * (2 * (int64_t)sizeof(float4) + (int64_t)sizeof(ilm_pixel));
     j->ctx = ctx;
     j->stage = stage_take(ctx, stage_bytes(wh));

@@ -18,7 +18,9 @@
  *   k_begin, k_send  a request's sums cleared; its results into pinned memory
  *
  * Every kernel reads its work count from device memory, so a whole chunk is a fixed launch
- * sequence (capturable as a hipGraph) that waits for nothing on the host between depths.
+ * sequence, capturable as a hipGraph, in which no depth waits for the host. (A chunk that is a
+ * call's only one leaves out the launches of depths that would find nothing to do: the host then
+ * follows the counts k_shade reports.)
  */
 #include "quad.h"
 

@@ -188,7 +188,8 @@ typedef struct ilm_opts {
     int32_t bvh_layout;         /* ILM_BVH_* (default FP32) */
     int32_t tri_test;           /* ILM_TRI_* (default Moller-Trumbore) */
     int64_t paths_in_flight;    /* 0 = automatic */
-    int64_t hbm_budget_bytes;   /* serving admission budget; 0 = 90% of free device memory */
+    int64_t hbm_budget_bytes;   /* serving admission budget; 0 = 90% of free device memory. A request is
+                                 * charged 56 bytes a pixel while admitted (its buffers take 36). */
     int32_t use_graphs;         /* capture the per-chunk pipeline as a hipGraph */
     int32_t max_queued;         /* serving: admission queue bound (0 = 4096) */
     int32_t extend_mode;        /* ILM_EXTEND_*: how extend waves schedule their rays */
@@ -265,7 +266,7 @@ typedef struct ilm_stats {
     double busy_ms;
     double p50_ms, p99_ms;      /* request latency: completion - submission */
     int64_t hbm_budget_bytes;
-    int64_t hbm_in_use_bytes;
+    int64_t hbm_in_use_bytes;   /* charged by the requests admitted now */
     uint64_t bvh_cache_hits;    /* meshes whose BVH came from the cache */
     uint64_t bvh_cache_misses;  /* meshes built (and stored) with a cache directory set */
 } ilm_stats;
