@@ -133,6 +133,25 @@ static hipError_t dupload(ilm_scene* s, T** dst, const T* src, size_t count) {
     return copy_sync(s->ctx, *dst, src, count * sizeof(T), hipMemcpyHostToDevice);
 }
 
+/* Two arrays in one allocation (the second 256-byte aligned), their copies waited for together: an
+ * allocation and a wait take some 15 us, which a scene of a few triangles spends its upload on. */
+template <class A, class B>
+static hipError_t dupload2(ilm_scene* s, A** da, const A* a, size_t na, B** db, const B* b, size_t nb) {
+    *da = nullptr;
+    *db = nullptr;
+    const size_t off = (na * sizeof(A) + 255) & ~(size_t)255;
+    char* p = nullptr;
+    hipError_t e = dalloc(s, (void**)&p, off + nb * sizeof(B));
+    if (e != hipSuccess || !p) return e;
+    if (na) *da = (A*)p;
+    if (nb) *db = (B*)(p + off);
+    const hipStream_t st = s->ctx->copy_stream;
+    if (na) e = hipMemcpyAsync(p, a, na * sizeof(A), hipMemcpyHostToDevice, st);
+    if (nb && e == hipSuccess) e = hipMemcpyAsync(p + off, b, nb * sizeof(B), hipMemcpyHostToDevice, st);
+    const hipError_t w = hipStreamSynchronize(st);   /* the first copy too when the second failed */
+    return e != hipSuccess ? e : w;
+}
+
 static int upload_texture(ilm_ctx* ctx, ilm_scene* s, const ilm_texture_desc& t, DTex& d) {
     std::memset(&d, 0, sizeof(d));
     d.type = t.type;
@@ -228,10 +247,6 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
     BuildOpts bo;
     for (int i = 0; i < d->num_meshes; i++) {
         const ilm_mesh_desc& m = d->meshes[i];
-        Box mb;
-        mb.reset();
-        for (int64_t k = 0; k < 3LL * m.num_triangles; k++) mb.grow(&m.positions[3 * m.indices[k]]);
-        mesh_bounds[i] = mb;
         MeshBVH bvh;
         bool cached = false;
         uint64_t key = 0;
@@ -252,7 +267,8 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
         s->quant_max_exp = std::max(s->quant_max_exp, qnodes_max_exponent(bvh.qnodes));
         /* The FNode layout and the shading vertices are made beside the rest of the mesh's upload, so
          * that a mesh whose other layouts come from the cache waits for neither: a cached upload of
-         * 722k triangles takes 62 to 66 ms (64.5 without FNodes, 86 with both made in turn). */
+         * 722k triangles takes 60 ms, of 101k 5.0 (64.7 and 4.9 without FNodes, 85 and 6.3 with both made
+         * in turn; 62 to 66 and 6.4 with the mesh's bounds taken before the threads start). */
         std::future<LayoutF> flayout = beside(m.num_triangles, [&bvh] { return make_layout_f(bvh.nodes, bvh.root); });
         /* shading vertices by original triangle index: the same floats the kernel would gather
          * through the index array */
@@ -266,6 +282,10 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
                 }
             return sv;
         });
+        Box mb;
+        mb.reset();
+        for (int64_t k = 0; k < 3LL * m.num_triangles; k++) mb.grow(&m.positions[3 * m.indices[k]]);
+        mesh_bounds[i] = mb;
         std::vector<float4> tris(3 * (size_t)m.num_triangles);
         for (int k = 0; k < m.num_triangles; k++) {
             int t = bvh.order[k];
@@ -292,12 +312,11 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
         if (!m.face_normals) HIPTRY(ctx, dupload(s.get(), &np, m.normals, 3 * (size_t)m.num_vertices));
         if (m.has_texcoords) HIPTRY(ctx, dupload(s.get(), &up, m.texcoords, 2 * (size_t)m.num_vertices));
         const LayoutF lf = flayout.get();
-        FNode* fn;
-        HIPTRY(ctx, dupload(s.get(), &fn, lf.nodes.data(), lf.nodes.size()));
         blas_flevels = std::max(blas_flevels, lf.levels);
         const std::vector<float4> sv = sverts.get();
+        FNode* fn;
         float4* svp;
-        HIPTRY(ctx, dupload(s.get(), &svp, sv.data(), sv.size()));
+        HIPTRY(ctx, dupload2(s.get(), &fn, lf.nodes.data(), lf.nodes.size(), &svp, sv.data(), sv.size()));
         dm.nodes = bn; dm.qnodes = qn; dm.tris = tp; dm.idx = ip; dm.pos = pp; dm.nrm = np; dm.uv = up;
         dm.svert = svp;
         dm.fnodes = fn;
@@ -391,12 +410,11 @@ int ilm_scene_upload(ilm_ctx* ctx, const ilm_scene_desc* d, ilm_scene** out) {
             for (int k = 0; k < 4; k++) n.child[k] = direct(n.child[k]);
         BNode* bn; QNode* qn;
         HIPTRY(ctx, dupload(s.get(), &bn, T2.nodes.data(), T2.nodes.size()));
-        HIPTRY(ctx, dupload(s.get(), &qn, TQ.nodes.data(), TQ.nodes.size()));
-        hs.tlas = bn; hs.qtlas = qn;
         hs.tlas_root = direct(T2.root);
         const LayoutF tf = make_layout_f(T2.nodes, hs.tlas_root);
         FNode* fn;
-        HIPTRY(ctx, dupload(s.get(), &fn, tf.nodes.data(), tf.nodes.size()));
+        HIPTRY(ctx, dupload2(s.get(), &fn, tf.nodes.data(), tf.nodes.size(), &qn, TQ.nodes.data(), TQ.nodes.size()));
+        hs.tlas = bn; hs.qtlas = qn;
         hs.ftlas = fn;
         hs.ftlas_root = tf.root;
         tlas_flevels = tf.levels;
